@@ -6,6 +6,7 @@
 // order by one workgroup per result.
 #include "dmk_internal.h"
 #include "mlp.h"
+#include "mlp_device.h"
 
 #include <hip/hip_runtime.h>
 
@@ -264,35 +265,16 @@ __device__ inline void features(double Di, double ri, double ui, double theta, d
 	f[2] = float(ui / rms_u);
 	f[3] = float(fmin(fmax(tols_unit, -10.0), 10.0));
 }
-
-__device__ inline float mlp_eval(const float* __restrict__ P, const float x[kMlpIn])
-{
-	float h1[kMlpHidden];
-#pragma unroll
-	for (int o = 0; o < kMlpHidden; ++o) {
-		float a = P[kMlpOffB1 + o];
-#pragma unroll
-		for (int i = 0; i < kMlpIn; ++i)
-			a += P[kMlpOffW1 + o * kMlpIn + i] * x[i];
-		h1[o] = tanhf(a);
-	}
-	float out = P[kMlpOffB3];
-	for (int o = 0; o < kMlpHidden; ++o) {
-		float a = P[kMlpOffB2 + o];
-#pragma unroll 16
-		for (int i = 0; i < kMlpHidden; ++i)
-			a += P[kMlpOffW2 + o * kMlpHidden + i] * h1[i];
-		out += P[kMlpOffW3 + o] * tanhf(a);
-	}
-	return out;
-}
 } // namespace
 
 // t_i = t_ols,i + MLP(features_i) * rms_r / sD: the network learns a correction on top of
 // Olsen's diagonal one, in units of rms_r / sD (its output layer starts at zero, so an
 // untrained network is exactly the diagonal method). eps = sums[0] / sums[1] from the Olsen
 // dot products of this iterate.
-__global__ __launch_bounds__(kDT) void precond_mlp_kernel(const float* __restrict__ params,
+//
+// A wave computes the features of 64 consecutive elements, one per lane, and evaluates them as
+// four 16-sample tiles on MFMAs (mlp_device.h).
+__global__ __launch_bounds__(kDT) __attribute__((amdgpu_waves_per_eu(2))) void precond_mlp_kernel(const float* __restrict__ params,
                                                           const double* __restrict__ r,
                                                           const double* __restrict__ u,
                                                           const double* __restrict__ D,
@@ -301,17 +283,36 @@ __global__ __launch_bounds__(kDT) void precond_mlp_kernel(const float* __restric
                                                           double sD, double rms_r, double rms_u,
                                                           int64_t n, double* __restrict__ t)
 {
-	__shared__ float P[kMlpParams];
-	for (int i = threadIdx.x; i < kMlpParams; i += kDT)
-		P[i] = params[i];
+	__shared__ __attribute__((aligned(16))) MlpSmall sm;
+	sm.load(params, threadIdx.x);
+	const int  lane = threadIdx.x & 63;
+	const int  c = lane & 15, g = lane >> 4;
+	MlpWeights w;
+	w.load(params, c, g);
 	__syncthreads();
-	const double eps  = (sums[1] != 0.0) ? sums[0] / sums[1] : 0.0;
-	const double unit = rms_r / sD;
-	for (int64_t i = int64_t(blockIdx.x) * kDT + threadIdx.x; i < n; i += int64_t(gridDim.x) * kDT) {
-		const double tols = olsen_elem(D[i], r[i], u[i], theta, floor_, eps);
-		float        f[kMlpIn];
+	const double  eps  = (sums[1] != 0.0) ? sums[0] / sums[1] : 0.0;
+	const double  unit = rms_r / sD;
+	const int64_t step = int64_t(gridDim.x) * kDT;
+	for (int64_t i0 = int64_t(blockIdx.x) * kDT + (threadIdx.x - lane); i0 < n; i0 += step) {
+		// Every lane of the wave takes part in the tiles: past the end it repeats the last element.
+		const int64_t i    = i0 + lane < n ? i0 + lane : n - 1;
+		const double  tols = olsen_elem(D[i], r[i], u[i], theta, floor_, eps);
+		float         f[kMlpIn];
 		features(D[i], r[i], u[i], theta, sD, rms_r, rms_u, tols / unit, f);
-		t[i] = tols + double(mlp_eval(P, f)) * unit;
+		float y = 0.0f;
+#pragma unroll 1
+		for (int q = 0; q < 4; ++q) {
+			mlp_tile_fence();
+			const int   src = kMlpTile * q + c;
+			const float f0 = __shfl(f[0], src), f1 = __shfl(f[1], src);
+			const float f2 = __shfl(f[2], src), f3 = __shfl(f[3], src);
+			const float xi = g == 0 ? f0 : g == 1 ? f1 : g == 2 ? f2 : f3;
+			const float out = mlp_forward_tile(w, sm, g, xi);
+			if (g == q)
+				y = out;
+		}
+		if (i0 + lane < n)
+			t[i] = tols + double(y) * unit;
 	}
 }
 
@@ -409,8 +410,8 @@ void launch_precond_mlp(const float* params, const double* r, const double* u, c
                         double rms_u, int64_t n, double* t, hipStream_t s)
 {
 	unsigned g = grid_n(n);
-	if (g > 2048)
-		g = 2048;
+	if (g > 512)
+		g = 512; // resident at once; the weights are loaded once per wave
 	hipLaunchKernelGGL(precond_mlp_kernel, dim3(g), dim3(kDT), 0, s, params, r, u, D, theta, floor_,
 	                   sums, sD, rms_r, rms_u, n, t);
 	DMK_HIP_CHECK(hipGetLastError());

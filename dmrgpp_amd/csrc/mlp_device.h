@@ -1,0 +1,181 @@
+// Device functions of the learned preconditioner's network (4 -> 64 -> 64 -> 1, tanh, FP32),
+// shared by its inference, training and Davidson kernels: one wave evaluates 16 samples at a
+// time on the matrix units.
+//
+// Lane l = 16 g + c holds, for sample c of the tile, the hidden units o = 16 b + 4 g + r (block
+// b < 4, register r < 4): the layout of the MFMA result D[4 g + r][c]. The same registers are the
+// right operand of the next layer as they stand, since a contraction may take its k in any order:
+// lane group g supplies its own units on the right and W2[o][those units] on the left. So nothing
+// goes through LDS between layers, and the whole W2 stays in registers.
+//
+// Inference multiplies layer 2 on bf16 MFMAs with every FP32 operand split exactly into three
+// bf16 parts (8 + 8 + 8 bits: h = bf16(v), m = bf16(v - h), l = v - h - m rounded) and the six
+// products down to 2^-17 of the leading one kept (l l, l m and m l, below 2^-25, are dropped),
+// accumulated in FP32. The reason is the issue port: on gfx950 an FP32 (or FP64) MFMA keeps the
+// vector ALU from issuing for its whole duration (32 MFMAs and 128 FMAs, two waves per SIMD: 1.85
+// and 1.04 ms alone, 2.65 ms together), a bf16 MFMA does not (1.83 and 1.04 ms alone, 1.85
+// together), and the tanh work alone keeps the vector ALU busy.
+#pragma once
+
+#include "mlp.h"
+
+#include <hip/hip_runtime.h>
+
+namespace dmk {
+
+typedef float  mlp_f4 __attribute__((ext_vector_type(4)));
+typedef __bf16 mlp_b8 __attribute__((ext_vector_type(8)));
+
+constexpr int kMlpTile   = 16;             // samples per wave and pass
+constexpr int kMlpBlocks = kMlpHidden / 16; // 16-unit blocks of a hidden layer
+
+__device__ inline mlp_f4 mlp_mma(float a, float b, mlp_f4 c)
+{
+	return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+__device__ inline mlp_f4 mlp_mma(mlp_b8 a, mlp_b8 b, mlp_f4 c)
+{
+	return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+}
+
+// Eight FP32 values as three bf16 parts each; the differences are exact.
+struct MlpSplit {
+	mlp_b8 h, m, l;
+	__device__ inline void set(int i, float v)
+	{
+		h[i]          = __bf16(v);
+		const float d = v - float(h[i]);
+		m[i]          = __bf16(d);
+		l[i]          = __bf16(d - float(m[i]));
+	}
+	// For any value: past the largest bf16 the rest goes to m and l; an infinity is that value.
+	__device__ inline void set_any(int i, float v)
+	{
+		const float top = 3.3895314e38f;
+		h[i]            = __bf16(v > top ? top : v < -top ? -top : v);
+		const float d   = isinf(v) ? 0.0f : v - float(h[i]);
+		m[i]            = __bf16(d);
+		l[i]            = __bf16(d - float(m[i]));
+	}
+};
+
+// tanh in FP32: x + x^3 P(x^2) below 0.6 (P: minimax polynomial of (tanh(x)/x - 1)/x^2, 3e-9),
+// 1 - 2 / (1 + exp(2 x)) from the hardware exp2 and reciprocal above. Absolute error at most
+// 2.2e-7, 0.8 units in the last place rms (over [-9, 9], exp2 one unit off);
+// +-1 at infinity, NaN for NaN. Both branches are computed: 12 vector operations and two
+// transcendental ones, without divergence.
+__device__ inline float mlp_tanh(float x)
+{
+	const float ax = fabsf(x);
+	const float t  = __builtin_amdgcn_exp2f(2.88539008f * x);
+	const float m  = __builtin_amdgcn_rcpf(1.0f + t);
+	const float s  = x * x;
+	float       p  = -5.89515828e-3f;
+	p              = fmaf(p, s, 2.07959712e-2f);
+	p              = fmaf(p, s, -5.37838303e-2f);
+	p              = fmaf(p, s, 1.33319244e-1f);
+	p              = fmaf(p, s, -3.33332986e-1f);
+	const float lo = fmaf(x * s, p, x);
+	const float hi = fmaf(-2.0f, m, 1.0f);
+	return ax < 0.6f ? lo : hi;
+}
+
+// The forward weights of one wave: left operands of both layers in registers; biases and W3
+// (which only depend on the lane group) are read from the workgroup's LDS copy per tile.
+struct MlpWeights {
+	float    w1[kMlpBlocks];    // W1[16 b + c][g]
+	MlpSplit w2[kMlpBlocks][2]; // [b2][s]: W2[16 b2 + c][k], k = 32 s + 16 (i / 4) + 4 g + i % 4
+
+	__device__ inline void load(const float* __restrict__ params, int c, int g)
+	{
+#pragma unroll
+		for (int b = 0; b < kMlpBlocks; ++b)
+			w1[b] = params[kMlpOffW1 + (16 * b + c) * kMlpIn + g];
+#pragma unroll
+		for (int b2 = 0; b2 < kMlpBlocks; ++b2)
+#pragma unroll
+			for (int s = 0; s < 2; ++s)
+#pragma unroll
+				for (int i = 0; i < 8; ++i)
+					w2[b2][s].set_any(i, params[kMlpOffW2 + (16 * b2 + c) * kMlpHidden + 32 * s
+					                        + 16 * (i >> 2) + 4 * g + (i & 3)]);
+	}
+};
+
+// Biases of both layers and the output layer, in LDS.
+struct MlpSmall {
+	float b1[kMlpHidden], b2[kMlpHidden], w3[kMlpHidden];
+	float b3;
+
+	// By the first 64 threads of the workgroup; a barrier must follow.
+	__device__ inline void load(const float* __restrict__ params, int tid)
+	{
+		if (tid < kMlpHidden) {
+			b1[tid] = params[kMlpOffB1 + tid];
+			b2[tid] = params[kMlpOffB2 + tid];
+			w3[tid] = params[kMlpOffW3 + tid];
+		}
+		if (tid == 0)
+			b3 = params[kMlpOffB3];
+	}
+	__device__ inline mlp_f4 at(const float* v, int b, int g) const
+	{
+		return *reinterpret_cast<const mlp_f4*>(v + 16 * b + 4 * g);
+	}
+};
+
+// Keeps the compiler from holding the LDS biases in registers across tiles (48 registers: with
+// W2's 64 they would leave three waves per SIMD, or spill).
+__device__ inline void mlp_tile_fence() { asm volatile("" ::: "memory"); }
+
+// The network's output for sample c of a tile (in every lane group); x is feature g of sample c.
+__device__ inline float mlp_forward_tile(const MlpWeights& w, const MlpSmall& sm, int g, float x)
+{
+	mlp_f4 h1[kMlpBlocks], h2[kMlpBlocks];
+#pragma unroll
+	for (int b = 0; b < kMlpBlocks; ++b) {
+		h1[b] = mlp_mma(w.w1[b], x, sm.at(sm.b1, b, g));
+		h2[b] = sm.at(sm.b2, b, g);
+	}
+#pragma unroll
+	for (int s = 0; s < 2; ++s) {
+		MlpSplit v;
+#pragma unroll
+		for (int i = 0; i < 8; ++i)
+			v.set(i, mlp_tanh(h1[2 * s + (i >> 2)][i & 3]));
+		// Small products first, and four independent accumulators between two uses of one.
+#pragma unroll
+		for (int b = 0; b < kMlpBlocks; ++b)
+			h2[b] = mlp_mma(w.w2[b][s].l, v.h, h2[b]);
+#pragma unroll
+		for (int b = 0; b < kMlpBlocks; ++b)
+			h2[b] = mlp_mma(w.w2[b][s].h, v.l, h2[b]);
+#pragma unroll
+		for (int b = 0; b < kMlpBlocks; ++b)
+			h2[b] = mlp_mma(w.w2[b][s].m, v.m, h2[b]);
+#pragma unroll
+		for (int b = 0; b < kMlpBlocks; ++b)
+			h2[b] = mlp_mma(w.w2[b][s].m, v.h, h2[b]);
+#pragma unroll
+		for (int b = 0; b < kMlpBlocks; ++b)
+			h2[b] = mlp_mma(w.w2[b][s].h, v.m, h2[b]);
+#pragma unroll
+		for (int b = 0; b < kMlpBlocks; ++b)
+			h2[b] = mlp_mma(w.w2[b][s].h, v.h, h2[b]);
+	}
+	float y = 0.0f;
+#pragma unroll
+	for (int b = 0; b < kMlpBlocks; ++b) {
+		const mlp_f4 w3 = sm.at(sm.w3, b, g);
+#pragma unroll
+		for (int r = 0; r < 4; ++r)
+			y = fmaf(w3[r], mlp_tanh(h2[b][r]), y);
+	}
+	// The sum over the four lane groups, the same in each.
+	y += __shfl_xor(y, 16);
+	y += __shfl_xor(y, 32);
+	return y + sm.b3;
+}
+
+} // namespace dmk

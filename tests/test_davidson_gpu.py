@@ -68,6 +68,31 @@ def test_gpu_mlp_forward_and_gradient_match_oracle():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("count", [1, 15, 16, 17, 63, 64, 65, 768 * 64 - 1, 768 * 64, 768 * 64 + 17])
+def test_gpu_mlp_forward_tiles(count):
+    """Every remainder of a 16-sample tile, a wave, a workgroup and the whole grid."""
+    rng = np.random.default_rng(count)
+    net = dm.Mlp(seed=5, capacity=1)
+    p = _params(rng).astype(np.float32)
+    net.set_params(p)
+    x = (3.0 * rng.standard_normal((count, 4))).astype(np.float32)
+    x[0] = [np.inf, -np.inf, 0.0, 1.0] if count > 64 else x[0]
+    y = net.forward(x)
+    # FP32 bound: 8 roundings in layer 1, 70 in layer 2 and the output, 4 units per tanh (at
+    # most 1); the split operands lose less than one more unit per product.
+    u = 2.0 ** -24
+    W1, b1, W2, b2, W3, b3 = mlp_oracle.unpack(p)
+    f = x[1:] if count > 64 else x
+    d1 = 8 * u * (np.abs(f.astype(np.float64)) @ np.abs(W1).T + np.abs(b1)) + 8 * u
+    d2 = d1 @ np.abs(W2).T + 70 * u * (np.abs(W2).sum(axis=1) + np.abs(b2)) + 8 * u
+    bound = d2 @ np.abs(W3) + 70 * u * (np.abs(W3).sum() + abs(b3))
+    want = mlp_oracle.forward(p.astype(np.float64), f.astype(np.float64))[0]
+    got = y[1:] if count > 64 else y
+    assert np.all(np.abs(got - want) <= bound)
+    net.close()
+
+
+@pytest.mark.gpu
 def test_gpu_mlp_training_reduces_loss():
     # Fit the clipped diagonal correction f3 = -f1 / f0 (a known function of the features).
     rng = np.random.default_rng(3)
