@@ -71,14 +71,21 @@ double Mlp::gradient(const float* x, const float* t, int64_t count, float* grad_
 {
 	if (count < 1 || !x || !t)
 		throw std::invalid_argument("mlp_gradient: empty batch");
+	if (!grad_host) {
+		float se = 0;
+		launch_mlp_loss(d_params_, x, t, count, d_part_, d_grad_, stream_);
+		DMK_HIP_CHECK(hipMemcpyAsync(&se, d_grad_ + kMlpParams, sizeof(float),
+		                             hipMemcpyDeviceToHost, stream_));
+		DMK_HIP_CHECK(hipStreamSynchronize(stream_));
+		return double(se) / double(count);
+	}
 	launch_mlp_grad(d_params_, x, t, count, d_part_, d_grad_, stream_);
 	std::vector<float> g(kMlpParams + 1);
 	DMK_HIP_CHECK(hipMemcpyAsync(g.data(), d_grad_, (kMlpParams + 1) * sizeof(float),
 	                             hipMemcpyDeviceToHost, stream_));
 	DMK_HIP_CHECK(hipStreamSynchronize(stream_));
-	if (grad_host)
-		for (int i = 0; i < kMlpParams; ++i)
-			grad_host[i] = g[size_t(i)];
+	for (int i = 0; i < kMlpParams; ++i)
+		grad_host[i] = g[size_t(i)];
 	return double(g[kMlpParams]) / double(count);
 }
 
@@ -103,9 +110,8 @@ void Mlp::train(int iters, int64_t batch, float lr, double* loss_last, double* l
 	for (int it = 0; it < iters; ++it) {
 		if (start + batch > count_)
 			start = 0;
-		launch_mlp_grad(d_params_, d_x_ + start * kMlpIn, d_t_ + start, batch, d_part_, d_grad_,
-		                stream_);
-		launch_mlp_adam(d_params_, d_grad_, d_m_, d_v_, lr, ++step_, stream_);
+		launch_mlp_train_step(d_params_, d_x_ + start * kMlpIn, d_t_ + start, batch, d_part_,
+		                      d_grad_, d_m_, d_v_, lr, ++step_, stream_);
 		start += batch;
 	}
 	float l = 0;

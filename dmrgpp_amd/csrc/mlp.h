@@ -22,8 +22,13 @@ constexpr int kMlpParams = kMlpOffB3 + 1; // 4545
 void launch_mlp_forward(const float* params, const float* x, int64_t count, float* y, hipStream_t s);
 void launch_mlp_grad(const float* params, const float* x, const float* t, int64_t count,
                      float* partial, float* grad, hipStream_t s);
-void launch_mlp_adam(float* params, const float* grad, float* m, float* v, float lr, int step,
-                     hipStream_t s);
+// The gradient and one Adam step (number `step` >= 1) on the parameters.
+void launch_mlp_train_step(float* params, const float* x, const float* t, int64_t count,
+                           float* partial, float* grad, float* m, float* v, float lr, int step,
+                           hipStream_t s);
+// The sum of squared errors into grad[kMlpParams].
+void launch_mlp_loss(const float* params, const float* x, const float* t, int64_t count,
+                     float* partial, float* grad, hipStream_t s);
 int  mlp_grad_parts(int64_t count);
 
 class Mlp {
@@ -38,7 +43,8 @@ public:
 	void         get_params(float* host) const;
 	void         set_params(const float* host);
 
-	// Gradient (host, kMlpParams) and mean squared error of the device batch (x, t).
+	// Gradient (host, kMlpParams) and mean squared error of the device batch (x, t); with a null
+	// gradient the error alone is computed.
 	double gradient(const float* x, const float* t, int64_t count, float* grad_host);
 
 	// Training set (device): count samples of kMlpIn features and one target.

@@ -93,6 +93,30 @@ def test_gpu_mlp_forward_tiles(count):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("count", [1, 15, 65, 256 * 64, 256 * 64 + 1, 3 * 256 * 64 - 5])
+def test_gpu_mlp_gradient_passes(count):
+    """Remainders of a tile and a pass, and one, two and three passes per workgroup; the loss alone
+    (after zero training steps) is the gradient call's."""
+    rng = np.random.default_rng(count)
+    net = dm.Mlp(seed=5, capacity=count)
+    p = _params(rng).astype(np.float32)
+    net.set_params(p)
+    x = rng.standard_normal((count, 4)).astype(np.float32)
+    t = rng.standard_normal(count).astype(np.float32)
+    g, loss = net.gradient(x, t)
+    want = mlp_oracle.gradient(p.astype(np.float64), x.astype(np.float64), t.astype(np.float64))
+    # FP32 sums: about 300 roundings on the way to a term, and the partial sums' own.
+    tol = 2.0 ** -24 * (300 + np.sqrt(count))
+    assert np.linalg.norm(g - want) <= tol * np.linalg.norm(want)
+    want_loss = mlp_oracle.loss(p, x, t)
+    assert abs(loss - want_loss) <= tol * want_loss
+    net.add_samples(x, t)
+    _, alone = net.train(0, batch=count)
+    assert abs(alone - want_loss) <= tol * want_loss
+    net.close()
+
+
+@pytest.mark.gpu
 def test_gpu_mlp_training_reduces_loss():
     # Fit the clipped diagonal correction f3 = -f1 / f0 (a known function of the features).
     rng = np.random.default_rng(3)
