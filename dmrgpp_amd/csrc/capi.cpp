@@ -410,7 +410,10 @@ int dmk_get_tuning(const dmk_handle* handle, dmk_tuning* tuning)
 	return guarded([&] {
 		if (!handle || !handle->plan || !tuning)
 			throw std::invalid_argument("dmk_get_tuning: null argument");
-		to_c(handle->plan->tuning(), tuning);
+		// Shapes that the rule picked are not reported: the caller gets the mode's base, in which
+		// any one value can be changed for dmk_set_tuning.
+		const dmk::Tuning& t = handle->plan->tuning();
+		to_c(t.by_rule ? dmk::default_tuning(handle->plan->precision()) : t, tuning);
 		return DMK_OK;
 	});
 }

@@ -805,20 +805,19 @@ Plan::Plan(int64_t noperator, int64_t npatches, const size_t* Lsz, const size_t*
 	d_prep_tiles_   = dev_alloc_copy(prep_tiles_);
 	d_prep_patches_ = dev_alloc_copy(prep_patches_);
 	// Per precision mode: a tuning the autotuner chose for this histogram earlier in the
-	// process, else the mode's default.
+	// process, else the rule's.
 	const int p0 = precision_;
 	for (int p = 0; p < 3; ++p) {
 		precision_     = p;
-		tuning_of_[p] = default_tuning(p);
+		tuning_of_[p] = rule_tuning(p);
 		cached_tuning(tuning_key(), tuning_of_[p]);
 	}
 	precision_ = p0;
 	retune(tuning_of_[p0]);
 }
 
-// The autotuner's usual choice per mode on the m = 2048 ladder superblocks: 64 x 64 tiles in the
-// XCD-aware order with split-k 2048 and two LDS stages (FP32 on 32 x 32 MFMA blocks); BF16x3
-// with 128 x 64 stage-2 tiles, split-k 1024.
+// 64 x 64 tiles in the XCD-aware order with split-k 2048 and two LDS stages (FP32 on 32 x 32 MFMA
+// blocks); BF16x3 with 128 x 64 stage-2 tiles, split-k 1024.
 Tuning default_tuning(int precision)
 {
 	Tuning t;
@@ -835,6 +834,177 @@ Tuning default_tuning(int precision)
 		t.depth  = 1;
 	}
 	return t;
+}
+
+// Launch shapes from t1 and t2, the numbers of 64 x 64 output tiles per CU of the two stages.
+// While the chip has only a few such tiles per CU, a launch is bounded by its longest tile's
+// chain of K chunks (each waits for its loads) and by idle CUs, so the smallest tiles with two
+// chunks in flight win by far; from a few tiles per CU on, operand traffic and per-tile overhead
+// count, and larger tiles with more residency (two LDS stages) win by less. Timed on Heisenberg
+// and Hubbard superblocks of m = 128 .. 3500 states, all tile shapes x split-k x load depths x
+// K chunks x MFMA forms; matvec in us with 64 x 64 tiles everywhere (the former choice), with the
+// rule, and with the best of all combinations:
+//            t1    t2    FP64                FP32                BF16x3
+//   spin 128   0.1  0.04    40 /   24 /   23    31 /   21 /   21    33 /   28 /   28
+//   spin 512   0.8  0.3     88 /   44 /   42    55 /   33 /   33    58 /   41 /   41
+//   Hub. 400   3.1  0.4    131 /   59 /   58    79 /   45 /   44    76 /   53 /   51
+//   spin 1024  4.5  0.8    254 /  185 /  182   145 /  110 /  105   106 /   84 /   84
+//   Hub. 1024  5.5  1.7    282 /  210 /  210   162 /  122 /  122   106 /   96 /   93
+//   spin 2048 17    3.1   1213 / 1130 / 1073   650 /  555 /  540   378 /  323 /  321
+//   Hub. 2048 24    3.6    969 /  895 /  865   526 /  470 /  451   352 /  303 /  299
+//   Hub. 3072 93    7.0   4323 / 4280 / 4218  2352 / 2200 / 2174  1501 / 1244 / 1244
+Tuning Plan::rule_tuning(int precision) const
+{
+	double t1 = 0, t2 = 0;
+	tiles_per_cu(&t1, &t2);
+	Tuning t;
+	t.by_rule = true;
+	t.xcd     = 1;
+	t.splitk  = 4096;
+	auto shape = [&](int bm1, int bn1, int bm2, int bn2, int depth, int kchunk) {
+		t.bm1    = bm1;
+		t.bn1    = bn1;
+		t.bm2    = bm2;
+		t.bn2    = bn2;
+		t.depth  = depth;
+		t.kchunk = kchunk;
+	};
+	if (precision == PREC_BF16X3) {
+		t.mfma32 = t2 < 2.5 ? 1 : 0;
+		t.splitk = t2 < 2.5 ? 2048 : 0;
+		if (t2 < 2.5)
+			shape(64, 64, 64, 64, 2, 1);
+		else
+			shape(128, 64, 128, 64, 1, 1);
+		return t;
+	}
+	// FP64 below t2 = 3 keeps the base tuning's order of summation (single K chunks, split-k 2048),
+	// so its results are the base tuning's bit for bit, whatever the tiles; a Davidson run that
+	// starts far from its state amplifies any difference. Up to 4 % slower there than free choice.
+	const bool f64 = precision == PREC_FP64;
+	if (f64) {
+		t.splitk = t2 < 3 ? 2048 : 4096;
+		if (t1 < 10 && t2 < 1.9)
+			shape(32, 32, 32, 32, 2, 1);
+		else if (t2 < 2.5)
+			shape(32, 64, 32, 32, 2, 1);
+		else if (t2 < 3)
+			shape(64, 32, 64, 32, 2, 1);
+		else if (t2 < 5)
+			shape(64, 32, 64, 32, 1, 2);
+		else
+			shape(64, 64, 64, 64, 1, 2);
+		return t;
+	}
+	if (t1 < 10 && t2 < 1.9) {
+		shape(32, 32, 32, 32, t1 < 4 ? 2 : 1, 1);
+		t.splitk = 2048;
+	} else if (t2 < 2.5) {
+		shape(64, 32, 32, 32, 1, 1);
+	} else if (t2 < 5) {
+		shape(64, 32, 32, 64, 1, 1);
+	} else {
+		shape(96, 64, 64, 64, 1, 1);
+		t.splitk = 0;
+	}
+	return t;
+}
+
+void Plan::tiles_per_cu(double* t1, double* t2) const
+{
+	auto tiles = [](const std::vector<PTask>& tasks) {
+		double n = 0;
+		for (const PTask& t : tasks)
+			n += double((t.m + 63) / 64) * double((t.n + 63) / 64);
+		return n / 256.0;
+	};
+	*t1 = tiles(t1_tasks_);
+	*t2 = tiles(t2_tasks_);
+}
+
+void Plan::release_multi_sets()
+{
+	for (TileSet& m : multi_sets_) {
+		pool_device_free(m.d1);
+		pool_device_free(m.d2);
+	}
+	multi_sets_.clear();
+}
+
+// With several vectors per launch the chip is filled sooner, and the larger tiles pay at smaller
+// problems. FP64, eight vectors, us per launch with the single vector's tiles / this rule's / the
+// best of all: Hubbard m = 400 (t2 0.4) 134 / 135 / 133, Heisenberg 1024 (0.8) 1392 / 1298 / 1242,
+// Hubbard 1400 (2.0) 2972 / 2537 / 2491, Hubbard 2048 (3.6) 7462 / 7138 / 7064.
+Plan::TileSet Plan::tile_set(int nvec)
+{
+	TileSet s;
+	s.bm1   = st1_.bm;
+	s.bn1   = st1_.bn;
+	s.bm2   = st2_.bm;
+	s.bn2   = st2_.bn;
+	s.depth = tuning_.depth;
+	s.d1    = st1_.d_tiles;
+	s.d2    = st2_.d_tiles;
+	s.n1    = int(st1_.tiles.size());
+	s.n2    = int(st2_.tiles.size());
+	if (nvec < 2 || !tuning_.by_rule)
+		return s;
+	double t1 = 0, t2 = 0;
+	tiles_per_cu(&t1, &t2);
+	t2 *= nvec;
+	TileSet w = s;
+	auto    tiles = [&](int bm, int bn) {
+                w.bm1 = std::max(w.bm1, bm);
+                w.bn1 = std::max(w.bn1, bn);
+                w.bm2 = std::max(w.bm2, bm);
+                w.bn2 = std::max(w.bn2, bn);
+	};
+	if (precision_ == PREC_BF16X3) {
+		if (t2 >= 2.5)
+			tiles(128, 64);
+	} else {
+		if (t2 >= 8)
+			tiles(64, 64);
+		else if (t2 >= 4)
+			tiles(64, 32);
+		// FP64 sums in the same order at either depth; FP32 folds its sums at one depth only.
+		if (precision_ == PREC_FP64 && t2 >= 4)
+			w.depth = tuning_.kchunk == 1 ? 2 : 1;
+	}
+	if (w.bm1 == s.bm1 && w.bn1 == s.bn1 && w.bm2 == s.bm2 && w.bn2 == s.bn2) {
+		s.depth = w.depth;
+		return s;
+	}
+	for (const TileSet& m : multi_sets_)
+		if (m.bm1 == w.bm1 && m.bn1 == w.bn1 && m.bm2 == w.bm2 && m.bn2 == w.bn2)
+			return m;
+	// The lists are uploaded on first use, which a stream capture cannot record: there the single
+	// vector's tiles serve.
+	hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+	DMK_HIP_CHECK(hipStreamIsCapturing(stream_, &cs));
+	if (cs != hipStreamCaptureStatusNone)
+		return s;
+	StageTables b1, b2;
+	b1.bm    = w.bm1;
+	b1.bn    = w.bn1;
+	b1.tasks = st1_.tasks;
+	b2.bm    = w.bm2;
+	b2.bn    = w.bn2;
+	b2.tasks = st2_.tasks;
+	build_tiles(b1, cost1_, tuning_.xcd);
+	build_tiles(b2, cost2s_, tuning_.xcd);
+	multi_sets_.reserve(multi_sets_.size() + 1);
+	w.n1 = int(b1.tiles.size());
+	w.n2 = int(b2.tiles.size());
+	w.d1 = dev_alloc_copy(b1.tiles);
+	try {
+		w.d2 = dev_alloc_copy(b2.tiles);
+	} catch (...) {
+		pool_device_free(w.d1);
+		throw;
+	}
+	multi_sets_.push_back(w);
+	return w;
 }
 
 std::string Plan::tuning_key() const
@@ -865,6 +1035,7 @@ Plan::~Plan()
 	pool_device_free(d_dg_);
 	st1_.release();
 	st2_.release();
+	release_multi_sets();
 	for (auto& e : ev_)
 		if (e)
 			(void)hipEventDestroy(e);
@@ -975,6 +1146,7 @@ void Plan::retune(const Tuning& t)
 	tuning_                 = t;
 	tuning_of_[precision_] = t;
 
+	release_multi_sets();
 	// Stage 1 as planned.
 	st1_.release();
 	st1_.bm    = t.bm1;
@@ -1063,6 +1235,7 @@ void Plan::retune(const Tuning& t)
 	}
 	stats_.ws_elems = ws;
 	build_tiles(st2_, cost, t.xcd);
+	cost2s_ = cost;
 	build_balanced(t);
 	chunks_.clear();
 	for (size_t r = 0; r < reduce_.size(); ++r)
@@ -1292,12 +1465,13 @@ void Plan::launch(const double* vin, int64_t ldin, double* vout, int64_t ldout, 
 	const int64_t  wss = stats_.ws_elems;
 	const int      npt = int(prep_tiles_.size());
 	const PStrides vs { xp_elems_, xt_elems_, bxs };
+	const TileSet  ts  = tile_set(nvec);
 	const int      v1  = tuning_.mfma32;
-	const int      dp  = tuning_.depth;
+	const int      dp  = ts.depth;
 	const int      kc  = tuning_.kchunk;
 	// Stage 2: one tile per workgroup, or the balanced persistent launch and its fix-up.
 	PanelLaunchExtra sk;
-	int              n2 = int(st2_.tiles.size());
+	int              n2 = ts.n2;
 	if (tuning_.persist) {
 		sk.items = d_sk_items_;
 		sk.bins  = d_sk_bins_;
@@ -1312,13 +1486,13 @@ void Plan::launch(const double* vin, int64_t ldin, double* vout, int64_t ldout, 
 		launch_prep_x<double>(d_prep_tiles_, npt, d_prep_patches_, vin, ldin, xp, xt, vs, nvec,
 		                      stream_);
 		const double* bases[PBASE_COUNT] = { d_apack_, d_bpack_, xp, xt, bx };
-		launch_panel_gemm<double, double>(st1_.bm, st1_.bn, 0, dp, kc, st1_.d_tasks, st1_.d_segs,
-		                                  st1_.d_tiles, int(st1_.tiles.size()), bases, vs, vout,
+		launch_panel_gemm<double, double>(ts.bm1, ts.bn1, 0, dp, kc, st1_.d_tasks, st1_.d_segs,
+		                                  ts.d1, ts.n1, bases, vs, vout,
 		                                  ldout, bx, bxs, nvec, 0, stream_);
 		if (mid)
 			DMK_HIP_CHECK(hipEventRecord(mid, stream_));
-		launch_panel_gemm<double, double>(st2_.bm, st2_.bn, 0, dp, kc, st2_.d_tasks, st2_.d_segs,
-		                                  st2_.d_tiles, n2, bases, vs, vout, ldout, ws, wss, nvec,
+		launch_panel_gemm<double, double>(ts.bm2, ts.bn2, 0, dp, kc, st2_.d_tasks, st2_.d_segs,
+		                                  ts.d2, n2, bases, vs, vout, ldout, ws, wss, nvec,
 		                                  beta, stream_, sk);
 		launch_splitk_reduce<double, double>(d_reduce_, d_chunks_, int(chunks_.size()), ws, wss,
 		                                     vout, ldout, nvec, beta, stream_);
@@ -1338,13 +1512,13 @@ void Plan::launch(const double* vin, int64_t ldin, double* vout, int64_t ldout, 
 		const void* hi[PBASE_COUNT] = { d_apack16_, d_bpack16_, xph, xth, bh };
 		const void* lo[PBASE_COUNT] = { d_apack16_ ? d_apack16_ + na : nullptr,
 			                        d_bpack16_ ? d_bpack16_ + nb : nullptr, xpl, xtl, bl };
-		launch_panel_bf16x3(st1_.bm, st1_.bn, v1, dp, st1_.d_tasks, st1_.d_segs, st1_.d_tiles,
-		                    int(st1_.tiles.size()), hi, lo, vs, vout, ldout, nullptr, bh, bl, bxs,
+		launch_panel_bf16x3(ts.bm1, ts.bn1, v1, dp, st1_.d_tasks, st1_.d_segs, ts.d1,
+		                    ts.n1, hi, lo, vs, vout, ldout, nullptr, bh, bl, bxs,
 		                    true, nvec, 0, stream_);
 		if (mid)
 			DMK_HIP_CHECK(hipEventRecord(mid, stream_));
 		float* ws = static_cast<float*>(d_ws);
-		launch_panel_bf16x3(st2_.bm, st2_.bn, v1, dp, st2_.d_tasks, st2_.d_segs, st2_.d_tiles, n2,
+		launch_panel_bf16x3(ts.bm2, ts.bn2, v1, dp, st2_.d_tasks, st2_.d_segs, ts.d2, n2,
 		                    hi, lo, vs, vout, ldout, ws, nullptr, nullptr, wss, false, nvec, beta,
 		                    stream_, sk);
 		launch_splitk_reduce<float, double>(d_reduce_, d_chunks_, int(chunks_.size()), ws, wss,
@@ -1359,13 +1533,13 @@ void Plan::launch(const double* vin, int64_t ldin, double* vout, int64_t ldout, 
 		launch_prep_x<float>(d_prep_tiles_, npt, d_prep_patches_, vin, ldin, xp, xt, vs, nvec,
 		                     stream_);
 		const float* bases[PBASE_COUNT] = { d_apack32_, d_bpack32_, xp, xt, bx };
-		launch_panel_gemm<float, float>(st1_.bm, st1_.bn, v1, dp, kc, st1_.d_tasks, st1_.d_segs,
-		                                st1_.d_tiles, int(st1_.tiles.size()), bases, vs, bx, bxs,
+		launch_panel_gemm<float, float>(ts.bm1, ts.bn1, v1, dp, kc, st1_.d_tasks, st1_.d_segs,
+		                                ts.d1, ts.n1, bases, vs, bx, bxs,
 		                                bx, bxs, nvec, 0, stream_);
 		if (mid)
 			DMK_HIP_CHECK(hipEventRecord(mid, stream_));
-		launch_panel_gemm<float, double>(st2_.bm, st2_.bn, v1, dp, kc, st2_.d_tasks, st2_.d_segs,
-		                                 st2_.d_tiles, n2, bases, vs, vout, ldout, ws, wss, nvec,
+		launch_panel_gemm<float, double>(ts.bm2, ts.bn2, v1, dp, kc, st2_.d_tasks, st2_.d_segs,
+		                                 ts.d2, n2, bases, vs, vout, ldout, ws, wss, nvec,
 		                                 beta, stream_, sk);
 		launch_splitk_reduce<float, double>(d_reduce_, d_chunks_, int(chunks_.size()), ws, wss,
 		                                    vout, ldout, nvec, beta, stream_);
@@ -1455,7 +1629,7 @@ Tuning Plan::autotune(const double* vin, double* vout, int iters)
 {
 	if (iters < 1)
 		throw std::invalid_argument("dmk_autotune: iters must be >= 1");
-	// Coordinate descent from the mode's default: each launch parameter in turn takes every
+	// Coordinate descent from the better of the mode's base and the rule's shapes: each launch parameter in turn takes every
 	// value with the others fixed, keeping the fastest; two passes.
 	auto time_of = [&](const Tuning& t) {
 		retune(t);
@@ -1468,6 +1642,16 @@ Tuning Plan::autotune(const double* vin, double* vout, int iters)
 	double best_ms = time_of(best);
 	// Every timed candidate, for the final re-timing of the leaders.
 	std::vector<std::pair<double, Tuning>> seen { { best_ms, best } };
+	{ // the rule's shapes are a second start
+		Tuning t  = rule_tuning(precision_);
+		t.by_rule = false;
+		const double ms = time_of(t);
+		seen.emplace_back(ms, t);
+		if (ms < best_ms) {
+			best_ms = ms;
+			best    = t;
+		}
+	}
 	auto try_set = [&](const std::vector<Tuning>& cands) {
 		for (const Tuning& t : cands) {
 			if (t == best)

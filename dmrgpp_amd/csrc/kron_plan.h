@@ -62,12 +62,14 @@ struct Tuning {
 	int depth  = 1; // global loads issued this many K chunks ahead (1 or 2)
 	int kchunk = 1; // K chunk depth in units of the mode's base chunk (1 or 2)
 	int persist = 0; // k > 0: stage 2 as a balanced persistent launch, k workgroups per CU at most
+	// Chosen by Plan::rule_tuning for the plan's problem (neither set nor autotuned).
+	bool by_rule = false;
 
 	bool operator==(const Tuning& o) const
 	{
 		return bm1 == o.bm1 && bn1 == o.bn1 && bm2 == o.bm2 && bn2 == o.bn2 && splitk == o.splitk
 		       && xcd == o.xcd && mfma32 == o.mfma32 && depth == o.depth && kchunk == o.kchunk
-		       && persist == o.persist;
+		       && persist == o.persist && by_rule == o.by_rule;
 	}
 };
 
@@ -84,7 +86,8 @@ struct StageTables {
 	void               release();
 };
 
-// The starting tuning of a precision mode (before any autotuning).
+// The base tuning of a precision mode: where the autotuner starts, and what a handle whose
+// launch shapes nobody chose reports.
 Tuning default_tuning(int precision);
 
 // Whether the present blocks (both factors non-null) live in device or managed memory: true when
@@ -136,6 +139,12 @@ public:
 	// the fastest; the choice is cached per block-size histogram signature for later plans.
 	Tuning autotune(const double* vin, double* vout, int iters);
 
+	// The launch shapes of a precision mode for this plan's problem, by a rule on the number of
+	// its output tiles.
+	Tuning rule_tuning(int precision) const;
+	// Numbers of 64 x 64 output tiles per CU of the two stages.
+	void tiles_per_cu(double* t1, double* t2) const;
+
 	// Signature of the block-size histogram (log2 bins of the stage-2 task shapes).
 	std::string histogram_key() const;
 	// The autotuner cache key: the histogram signature and the precision mode.
@@ -170,6 +179,22 @@ private:
 	PlanStats   stats_;
 	StageTables st1_, st2_;
 	hipStream_t stream_ = nullptr;
+
+	// Tile lists of the launches for several vectors, for the rule's tilings that differ from the
+	// single vector's (Plan::tile_set); built on first use, dropped by retune.
+	struct TileSet {
+		int   bm1 = 0, bn1 = 0, bm2 = 0, bn2 = 0, depth = 1;
+		Tile* d1 = nullptr;
+		Tile* d2 = nullptr;
+		int   n1 = 0, n2 = 0;
+	};
+	std::vector<TileSet> multi_sets_;
+	std::vector<double>  cost2s_; // cost of st2_'s (split) tasks
+	// The tiling of a launch for nvec vectors: the current tuning's, or for a rule-chosen tuning
+	// the one that suits nvec times as many tiles. Only tile shapes and load depth vary, not the
+	// order in which any element is summed, so a vector's result does not depend on nvec.
+	TileSet tile_set(int nvec);
+	void    release_multi_sets();
 
 	// Unsplit tasks of both stages as planned from the blocks (retune builds the tables).
 	std::vector<PTask>  t1_tasks_, t2_tasks_;

@@ -47,6 +47,7 @@ namespace dmk {
 namespace {
 
 constexpr int kPThreads = 256;
+constexpr int kFoldK    = 512; // elements of k per first-level sum
 
 typedef double d2_t __attribute__((ext_vector_type(2)));
 typedef float  f4_t __attribute__((ext_vector_type(4)));
@@ -321,6 +322,15 @@ __global__ __launch_bounds__(kPThreads) void panel_gemm_kernel(
 	constexpr int NW = LA::NI + LB::NI;      // LDS-DMA instructions per wave per chunk
 	static_assert(NF % VW == 0, "fragment / vector mismatch");
 	static_assert(NS == 2 || NS == 3, "two or three stages");
+	// FP32 sums longer than kFoldK are kept in two levels: the MFMA accumulators are added to a
+	// second set and cleared about every kFoldK elements of k, so the rounding error of a long
+	// contraction does not grow with its length (m = 2048 ladder, K to 7410 in one or two pieces:
+	// error against 64 bits 1.3e-6 without, 4.8e-7 with, 9e-7 with split-k 2048 alone, whose
+	// partial sums cost 8 % of the stage). A few vector additions per 512 k; with two LDS stages and
+	// up to 64 x 64 tiles only, the launches of long sums (with three stages the 32 x 32 kernel
+	// lost 3 %, the 96 x 64 one 10 %, and the FP64 ones up to 10 %).
+	constexpr bool kFold      = std::is_same<T, float>::value && NS == 2 && BM <= 64 && BN <= 64;
+	constexpr int  kFoldSteps = kFoldK / (BK * NS) > 0 ? kFoldK / (BK * NS) : 1;
 
 	__shared__ vec_t A0[BM * VPR], B0[BN * VPR], A1[BM * VPR], B1[BN * VPR];
 	__shared__ vec_t A2[NS == 3 ? BM * VPR : 1], B2[NS == 3 ? BN * VPR : 1];
@@ -363,12 +373,25 @@ __global__ __launch_bounds__(kPThreads) void panel_gemm_kernel(
 			continue; // padding slot of the XCD-aware order
 		const PTask tk = load_const(tasks, tl.task);
 
-		acc_t acc[FI][FJ];
+		acc_t acc[FI][FJ], sum[kFold ? FI : 1][kFold ? FJ : 1];
 #pragma unroll
 		for (int i = 0; i < FI; ++i)
 #pragma unroll
-			for (int j = 0; j < FJ; ++j)
+			for (int j = 0; j < FJ; ++j) {
 				acc[i][j] = acc_t {};
+				if constexpr (kFold)
+					sum[i][j] = acc_t {};
+			}
+		auto fold = [&]() {
+			if constexpr (kFold)
+#pragma unroll
+				for (int i = 0; i < FI; ++i)
+#pragma unroll
+					for (int j = 0; j < FJ; ++j) {
+						sum[i][j] += acc[i][j];
+						acc[i][j] = acc_t {};
+					}
+		};
 
 		// The item's first chunk: `skip` whole chunks into the task's segments (with k > 0).
 		int seg = tk.seg_begin;
@@ -447,8 +470,12 @@ __global__ __launch_bounds__(kPThreads) void panel_gemm_kernel(
 				issue(A0, B0);
 				wait_vm_lgkm0<0>();
 				barrier_no_fence();
-				int c = 0;
+				int c = 0, left = kFoldSteps;
 				for (; c + 2 <= nch; c += 2) {
+					if (kFold && --left < 0) {
+						fold();
+						left = kFoldSteps - 1;
+					}
 					issue(A1, B1);
 					compute(A0, B0);
 					wait_vm_lgkm0<0>();
@@ -471,8 +498,12 @@ __global__ __launch_bounds__(kPThreads) void panel_gemm_kernel(
 				issue(A1, B1);
 				wait_vm_lgkm0<NW>();
 				barrier_no_fence();
-				int c = 0;
+				int c = 0, left = kFoldSteps;
 				for (; c + 3 <= nch; c += 3) {
+					if (kFold && --left < 0) {
+						fold();
+						left = kFoldSteps - 1;
+					}
 					issue(A2, B2);
 					compute(A0, B0);
 					wait_vm_lgkm0<NW>();
@@ -498,6 +529,12 @@ __global__ __launch_bounds__(kPThreads) void panel_gemm_kernel(
 			}
 			// Every load has landed before the stages are reused or the workgroup ends.
 			wait_vm_lgkm0<0>();
+			if constexpr (kFold)
+#pragma unroll
+				for (int i = 0; i < FI; ++i)
+#pragma unroll
+					for (int j = 0; j < FJ; ++j)
+						acc[i][j] += sum[i][j];
 		}
 
 		if (slot >= 0) {

@@ -198,12 +198,15 @@ int dmk_get_info(const dmk_handle* handle, dmk_info* info);
 /* Tuning of the launches. No reference counterpart (the Kokkos path hard-codes its shape,
  * BatchedGemmKokkos.h:110-130). dmk_set_tuning rebuilds the launch tables. A tuning belongs to
  * the handle's current precision mode: dmk_set_precision switches to the tuning last set or
- * autotuned for the selected mode (else the cached or the default one). */
+ * autotuned for the selected mode (else the cached one, else shapes that a rule picks for the
+ * problem's block sizes). While the rule's shapes are in use, dmk_get_tuning gives the mode's
+ * base tuning, a valid starting point for dmk_set_tuning; dmk_info counts what runs. */
 int dmk_get_tuning(const dmk_handle* handle, dmk_tuning* tuning);
 int dmk_set_tuning(dmk_handle* handle, const dmk_tuning* tuning);
 
 /* Tunes the launch shape on this handle's problem (iters matvecs per candidate, in the current
- * precision, on the device vectors vin/vout): coordinate descent from the mode's default over the
+ * precision, on the device vectors vin/vout): coordinate descent from the better of the mode's base
+ * tuning and the rule's shapes over the
  * MFMA form, load depth, stage-2 tile, split-k, tile order and stage-1 tile, two passes, keeping
  * the fastest. The choice is cached in the
  * process under the block-size histogram of the problem, and handles created later for a
