@@ -149,6 +149,33 @@ __device__ inline int64_t out_addr(const PTask& tk, int r, int c)
 	return tk.coff + int64_t(rr) * tk.sm + int64_t(blk) * tk.n + c;
 }
 
+// Walks the rows of a lane's output elements: offset of (row, column 0) from the task's coff as
+// out_addr gives it, with one division per start instead of two per element (the vector ALU and
+// the FP32 / FP64 MFMAs share the issue port: the divisions of a stage-1 tile took 10 % of the
+// FP32 launch).
+struct RowWalk {
+	int     rsplit, rr;
+	int64_t off, sm, wrap; // wrap: what leaving a block of rsplit rows adds
+	__device__ inline RowWalk(const PTask& tk, int row)
+	{
+		rsplit        = tk.rsplit;
+		sm            = tk.sm;
+		wrap          = int64_t(tk.n) - int64_t(tk.rsplit) * tk.sm;
+		const int blk = rsplit >= tk.m ? 0 : int(unsigned(row) / unsigned(rsplit));
+		rr            = row - blk * rsplit;
+		off           = tk.coff + int64_t(rr) * tk.sm + int64_t(blk) * tk.n;
+	}
+	__device__ inline void advance(int step)
+	{
+		rr += step;
+		off += step * sm;
+		while (rr >= rsplit) {
+			rr -= rsplit;
+			off += wrap;
+		}
+	}
+};
+
 // Element i of a descriptor array, read through the constant address space: scalar loads, which
 // an LDS-DMA load in flight (a vector memory operation that writes memory) does not make wait.
 template <typename S> __device__ inline S load_const(const S* p, int i)
@@ -197,19 +224,24 @@ template <typename E, int ROWS, int BK> struct TileLoad {
 	static constexpr int VW  = 16 / int(sizeof(E));
 	static constexpr int VPR = BK / VW;
 	static_assert(ROWS * VPR % kPThreads == 0, "tile / thread mismatch");
-	// Slot of vector kv of LDS row r. A 16-byte LDS access is served 8 lanes (32 banks) or 16
-	// lanes (64 banks) per pass; the fragment reads put consecutive rows on consecutive lanes,
-	// so the XOR mask f(r) keeps any 8 consecutive rows, and any 16 consecutive rows that start
-	// on the same bank, on distinct slots: f is a permutation of 0..VPR-1 on rows 8a..8a+7, on
-	// the even and on the odd rows of 16a..16a+15 (VPR = 8), and on each residue class mod 2
-	// within 8 rows and mod 4 within 16 rows (VPR = 4).
+	// Slot of vector kv of LDS row r. A 16-byte LDS read is served 16 lanes (256 bytes) per pass,
+	// and the passes take lanes {0-3, 12-15, 20-23, 24-27} and {4-11, 16-19, 28-31} of each half
+	// of the wave (the grouping that explains which of the former masks had conflicts in the
+	// counters and which had none). In the fragment reads lane l holds row l % 16 of vector group
+	// l / 16 (or row l % 32), so with q = r / 4 a pass mixes q = 0, 3 of one group with q = 1, 2 of
+	// the next, whose kv differs by the group stride; the mask (-q) mod 4 (VPR = 4, and times 4
+	// plus r mod 4 for VPR = 16, group stride 4) keeps all 16 on distinct slots, as does the one
+	// for VPR = 8 (group stride 2). With r mod 16 (VPR = 16) and (r / 2 mod 4) ^ (r / 8 mod 2)
+	// (VPR = 4) the FP64 double-chunk and BF16x3 kernels lost 13 to 16 % of the LDS cycles.
 	__device__ static inline int slot(int r, int kv)
 	{
 		int f;
-		if constexpr (VPR == 8)
+		if constexpr (VPR == 16)
+			f = (r & 3) | ((-(r >> 2) & 3) << 2);
+		else if constexpr (VPR == 8)
 			f = (r & 7) ^ ((r >> 3) & 1);
 		else if constexpr (VPR == 4)
-			f = ((r >> 1) & 3) ^ ((r >> 3) & 1);
+			f = -(r >> 2) & 3;
 		else
 			f = r & (VPR - 1);
 		return kv ^ f;
@@ -480,16 +512,16 @@ __global__ __launch_bounds__(kPThreads) void panel_gemm_kernel(
 					compute(A0, B0);
 					wait_vm_lgkm0<0>();
 					barrier_no_fence();
-					if (c + 2 == nch) {
-						compute(A1, B1);
-						break;
-					}
-					issue(A0, B0);
+					// One exit only: with a second one out of the middle of the loop the compiler
+					// kept the accumulators in two register sets and copied them, behind a wait
+					// for the last MFMA, in every round.
+					if (c + 2 < nch)
+						issue(A0, B0);
 					compute(A1, B1);
 					wait_vm_lgkm0<0>();
 					barrier_no_fence();
 				}
-				if (c + 1 == nch)
+				if (c < nch)
 					compute(A0, B0);
 			} else {
 				// At the top of each step stage 0 holds chunk c and chunk c+1 is in flight to
@@ -550,16 +582,25 @@ __global__ __launch_bounds__(kPThreads) void panel_gemm_kernel(
 						    acc[i][j][r];
 		} else {
 			const bool to_y = tk.out_is_y != 0;
+			const int  col0 = tl.n0 + wn + lr;
 #pragma unroll
-			for (int i = 0; i < FI; ++i)
+			for (int i = 0; i < FI; ++i) {
+				int     row = tl.m0 + wm + Op::kM * i + Op::row(lane, 0);
+				RowWalk w(tk, row);
 #pragma unroll
-				for (int j = 0; j < FJ; ++j)
+				for (int r = 0; r < Op::kRegs; ++r) {
+					if (r > 0) {
+						const int step = Op::row(0, r) - Op::row(0, r - 1);
+						row += step;
+						w.advance(step);
+					}
+					if (row >= tk.m)
+						break;
 #pragma unroll
-					for (int r = 0; r < Op::kRegs; ++r) {
-						const int row = tl.m0 + wm + Op::kM * i + Op::row(lane, r);
-						const int col = tl.n0 + wn + Op::kM * j + lr;
-						if (row < tk.m && col < tk.n) {
-							const int64_t addr = out_addr(tk, row, col);
+					for (int j = 0; j < FJ; ++j) {
+						const int col = col0 + Op::kM * j;
+						if (col < tk.n) {
+							const int64_t addr = w.off + col;
 							if (to_y) {
 								TO v = TO(acc[i][j][r]);
 								if (beta)
@@ -570,6 +611,8 @@ __global__ __launch_bounds__(kPThreads) void panel_gemm_kernel(
 							}
 						}
 					}
+				}
+			}
 		}
 		// The next item's first stores go to LDS buffer 0, which the last chunk may have used.
 		__syncthreads();
@@ -748,16 +791,13 @@ __global__ __launch_bounds__(kPThreads) void panel_bf16x3_kernel(
 					compute(S0);
 					wait_vm_lgkm0<0>();
 					barrier_no_fence();
-					if (c + 2 == nch) {
-						compute(S1);
-						break;
-					}
-					issue(S0);
+					if (c + 2 < nch) // one exit only, as in panel_gemm_kernel
+						issue(S0);
 					compute(S1);
 					wait_vm_lgkm0<0>();
 					barrier_no_fence();
 				}
-				if (c + 1 == nch)
+				if (c < nch)
 					compute(S0);
 			} else {
 				issue(S0);
@@ -804,16 +844,25 @@ __global__ __launch_bounds__(kPThreads) void panel_bf16x3_kernel(
 						    acc[i][j][r];
 		} else {
 			const bool to_y = tk.out_is_y != 0;
+			const int  col0 = tl.n0 + wn + lr;
 #pragma unroll
-			for (int i = 0; i < FI; ++i)
+			for (int i = 0; i < FI; ++i) {
+				int     row = tl.m0 + wm + Op::kM * i + Op::row(lane, 0);
+				RowWalk w(tk, row);
 #pragma unroll
-				for (int j = 0; j < FJ; ++j)
+				for (int r = 0; r < Op::kRegs; ++r) {
+					if (r > 0) {
+						const int step = Op::row(0, r) - Op::row(0, r - 1);
+						row += step;
+						w.advance(step);
+					}
+					if (row >= tk.m)
+						break;
 #pragma unroll
-					for (int r = 0; r < Op::kRegs; ++r) {
-						const int row = tl.m0 + wm + Op::kM * i + Op::row(lane, r);
-						const int col = tl.n0 + wn + Op::kM * j + lr;
-						if (row < tk.m && col < tk.n) {
-							const int64_t addr = out_addr(tk, row, col);
+					for (int j = 0; j < FJ; ++j) {
+						const int col = col0 + Op::kM * j;
+						if (col < tk.n) {
+							const int64_t addr = w.off + col;
 							const float   v    = acc[i][j][r];
 							if (to_y) {
 								double y = double(v);
@@ -829,6 +878,8 @@ __global__ __launch_bounds__(kPThreads) void panel_bf16x3_kernel(
 							}
 						}
 					}
+				}
+			}
 		}
 		__syncthreads(); // LDS buffer 0 is reused by the next item
 	}
