@@ -1,24 +1,20 @@
-// Variable-size batched GEMM: dmrg_Xgemm_vbatch (GPUPlugin/dmrg_vbatch.cpp:129-652) on the
-// K-major panel kernel of the matvec (panel_kernels.hip).
+// Variable-size batched GEMM: dmrg_Xgemm_vbatch (GPUPlugin/dmrg_vbatch.cpp:129-652) on FP64
+// MFMAs.
 //
 // The reference expands its groups into per-entry arrays and hands them to MAGMA
-// *_vbatched_max_nocheck (or a BLAS loop). Here every entry becomes one task of the panel
-// kernel (two for complex scalars), after its operands are staged into one workspace in the
-// panel kernel's K-major layout: the task computes C^T = op(B)^T op(A)^T, whose left operand is
-// op(B) column major (each column contiguous along k) and whose right operand is op(A)^T column
-// major (each row of op(A) contiguous along k), both with leading dimensions padded to a
-// multiple of kPanelPad and zero filled; C^T written by rows is C by columns. Staging makes transposes, conjugation and
-// complex scalars a property of the copy, so the GEMM launch only ever sees real K-major
-// operands, addressed as offsets into one allocation. Complex products run as real ones:
-//   Re C = Ar Br + (-Ai) Bi,   Im C = Ar Bi + Ai Br   (two segments per task).
-// The scatter then forms alpha W + beta C in the caller's C (C is not read when beta == 0, as
-// in BLAS). The call is synchronous, like the reference's.
+// *_vbatched_max_nocheck (or a BLAS loop). Here one launch computes the output tiles of all
+// entries straight from the caller's matrices (vbatch_kernels.hip); the host checks the
+// arguments and uploads the entries and the XCDs' tile lists in one copy. A batch in which some C overlaps an
+// operand's memory is computed into a workspace and copied back. The call is synchronous, like
+// the reference's.
 #include "vbatch.h"
 
 #include "dmk_internal.h"
 #include "pool.h"
 
 #include <algorithm>
+#include <cstdint>
+#include <cstring>
 #include <numeric>
 #include <stdexcept>
 #include <string>
@@ -26,21 +22,7 @@
 
 namespace dmk {
 
-template <typename T, typename TO>
-void launch_panel_gemm(int bm, int bn, int variant, int depth, int kchunk, const PTask* tasks,
-                       const PSeg* segs, const Tile* tiles, int ntiles, const T* const* bases,
-                       const PStrides& vs, TO* out_y, int64_t ystride, T* out_ws,
-                       int64_t wsstride, int nvec, int beta, hipStream_t stream,
-                       const PanelLaunchExtra& ex = PanelLaunchExtra {});
-
 namespace {
-
-struct Entry {
-	int           m, n, k, lda, ldb, ldc;
-	const double* a;
-	const double* b;
-	double*       c;
-};
 
 // op code of a BLAS transpose character: 0 = N, 1 = T, 2 = C (conjugate transpose).
 int trans_code(char t, const char* which)
@@ -60,39 +42,81 @@ int trans_code(char t, const char* which)
 	}
 }
 
-constexpr int64_t kChunk = 8192; // elements per staging / scatter workgroup (32 per thread)
+constexpr int kXcds = 8;
 
-// Appends copy jobs staging op(X) (rows x cols) from src into the workspace at dst, column
-// major with the leading dimension padded (panel_ld(rows)) and the padding zero filled.
-// Returns the staged size in elements.
-int64_t stage(std::vector<VbCopy>& jobs, const double* src, int ld, int rows, int cols,
-              int64_t dst, int flags)
+// Whether any output's memory range meets any input's (by range: interleaved submatrices count).
+bool outputs_meet_inputs(const std::vector<VbEntry>& ents, int ta, int tb, size_t scalar)
 {
-	const int     ldd   = int(panel_ld(rows));
-	const int64_t total = int64_t(ldd) * cols;
-	for (int64_t s = 0; s < total; s += kChunk) {
-		VbCopy j{};
-		j.src   = src;
-		j.dst   = dst;
-		j.start = s;
-		j.len   = std::min(kChunk, total - s);
-		j.rows  = rows;
-		j.ld    = ld;
-		j.flags = flags;
-		j.ldd   = ldd;
-		jobs.push_back(j);
+	struct Range {
+		uintptr_t lo, hi;
+		bool      out;
+	};
+	std::vector<Range> r;
+	r.reserve(3 * ents.size());
+	auto add = [&](const double* p, int rows, int cols, int ld, bool out) {
+		const uintptr_t lo = reinterpret_cast<uintptr_t>(p);
+		r.push_back(Range { lo, lo + (size_t(cols - 1) * size_t(ld) + size_t(rows)) * scalar, out });
+	};
+	for (const VbEntry& e : ents) {
+		add(e.c, e.m, e.n, e.ldc, true);
+		if (e.k > 0) {
+			add(e.a, ta ? e.k : e.m, ta ? e.m : e.k, e.lda, false);
+			add(e.b, tb ? e.n : e.k, tb ? e.k : e.n, e.ldb, false);
+		}
 	}
-	return total;
+	std::sort(r.begin(), r.end(), [](const Range& x, const Range& y) { return x.lo < y.lo; });
+	uintptr_t end[2] = { 0, 0 };
+	for (const Range& x : r) {
+		if (x.lo < end[x.out ? 0 : 1])
+			return true;
+		end[x.out ? 1 : 0] = std::max(end[x.out ? 1 : 0], x.hi);
+	}
+	return false;
 }
 
-template <typename T> T* upload(const std::vector<T>& v, std::vector<void*>& owned)
+// Which tiles each XCD's workgroups take (workgroup b runs on XCD b % 8): every entry's tiles, the
+// longest contractions first, in eight runs, so that neighbouring tiles share an L2; small entries
+// go whole to the XCD with the least work. The workgroups find their tiles in these lists, which
+// spares the host and the upload the tiles themselves (a few thousand per call).
+struct RunLists {
+	std::vector<VbRun> runs; // kXcds lists of nruns
+	int                nruns   = 0;
+	int64_t            longest = 0;
+};
+
+RunLists list_runs(const std::vector<VbEntry>& ents, int T)
 {
-	if (v.empty())
-		return nullptr;
-	void* p = pool_device_alloc(v.size() * sizeof(T));
-	owned.push_back(p);
-	DMK_HIP_CHECK(hipMemcpy(p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice));
-	return static_cast<T*>(p);
+	std::vector<int> order(ents.size());
+	std::iota(order.begin(), order.end(), 0);
+	std::stable_sort(order.begin(), order.end(),
+	                 [&](int x, int y) { return ents[size_t(x)].k > ents[size_t(y)].k; });
+	std::vector<VbRun> lists[kXcds];
+	double             load[kXcds] = {};
+	int64_t            count[kXcds] = {};
+	for (int e : order) {
+		const VbEntry& en   = ents[size_t(e)];
+		const int64_t  nt   = int64_t((en.m + T - 1) / T) * ((en.n + T - 1) / T);
+		const double   cost = double(en.k) + 32.0;
+		for (int64_t run = 0, t = 0; t < nt; ++run) {
+			const int64_t end = nt < kXcds ? nt : nt * (run + 1) / kXcds;
+			if (end == t)
+				continue;
+			const int x = int(std::min_element(load, load + kXcds) - load);
+			lists[x].push_back(VbRun { int32_t(count[x]), e, int32_t(t), int32_t(end) });
+			count[x] += end - t;
+			load[x] += cost * double(end - t);
+			t = end;
+		}
+	}
+	RunLists out;
+	for (int x = 0; x < kXcds; ++x) {
+		out.nruns   = std::max(out.nruns, int(lists[x].size()));
+		out.longest = std::max(out.longest, count[x]);
+	}
+	out.runs.assign(size_t(out.nruns) * kXcds, VbRun { INT32_MAX, 0, 0, 0 });
+	for (int x = 0; x < kXcds; ++x)
+		std::copy(lists[x].begin(), lists[x].end(), out.runs.begin() + size_t(x) * size_t(out.nruns));
+	return out;
 }
 
 } // namespace
@@ -108,7 +132,7 @@ void gemm_vbatch(bool cplx, char transa, char transb, const int* m, const int* n
 		return;
 	if (!m || !n || !k || !alpha || !a || !lda || !b || !ldb || !beta || !c || !ldc || !group_size)
 		throw std::invalid_argument("gemm_vbatch: null argument");
-	std::vector<Entry> ents;
+	std::vector<VbEntry> ents;
 	size_t             idx = 0;
 	for (size_t g = 0; g < group_count; ++g) {
 		if (group_size[g] < 0 || m[g] < 0 || n[g] < 0 || k[g] < 0)
@@ -119,7 +143,8 @@ void gemm_vbatch(bool cplx, char transa, char transb, const int* m, const int* n
 			throw std::invalid_argument("gemm_vbatch: leading dimension too small in group "
 			                            + std::to_string(g));
 		for (int i = 0; i < group_size[g]; ++i, ++idx) {
-			Entry e{ m[g], n[g], k[g], lda[g], ldb[g], ldc[g], a[idx], b[idx], c[idx] };
+			VbEntry e { a[idx], b[idx], c[idx], c[idx], m[g], n[g], k[g], lda[g], ldb[g], ldc[g],
+				    ldc[g], 0 };
 			if (e.m == 0 || e.n == 0)
 				continue;
 			if (!e.c || (e.k > 0 && (!e.a || !e.b)))
@@ -130,167 +155,74 @@ void gemm_vbatch(bool cplx, char transa, char transb, const int* m, const int* n
 	}
 	if (ents.empty())
 		return;
-	const bool alpha_zero = alpha[0] == 0.0 && (!cplx || alpha[1] == 0.0);
-	const bool beta_zero  = beta[0] == 0.0 && (!cplx || beta[1] == 0.0);
-	const int  cx         = cplx ? VB_CPLX : 0;
-
-	std::vector<VbCopy> copies;
-	std::vector<VbOut>  outs;
-	std::vector<PTask>  tasks;
-	std::vector<PSeg>   segs;
-	std::vector<double> cost;
-	int64_t             wsz = 0, csz = 0;
-	// Segment of C^T(n x m) += L(n x k) R(k x m): L = staged op(B) part at lo, R = staged
-	// op(A)^T part at ro, both K-major with leading dimension panel_ld(k).
-	auto seg = [&](int64_t lo, int64_t ro, int kk) {
-		PSeg s{};
-		s.loff  = lo;
-		s.roff  = ro;
-		s.lbase = PBASE_APACK;
-		s.rbase = PBASE_APACK;
-		s.ldl   = int32_t(panel_ld(kk));
-		s.ldr   = int32_t(panel_ld(kk));
-		s.k     = kk;
-		segs.push_back(s);
-	};
-	// Task C^T (n x m) written by rows of length m: element (j, i) at coff + i + j m, i.e. C
-	// (m x n) column major at coff.
-	auto task = [&](int64_t coff, int mm, int nn, int kk, int sb, int se) {
-		PTask t{};
-		t.coff      = coff;
-		t.m         = nn;
-		t.n         = mm;
-		t.rsplit    = nn;
-		t.sm        = mm;
-		t.seg_begin = sb;
-		t.seg_end   = se;
-		t.out_is_y  = 1;
-		tasks.push_back(t);
-		cost.push_back(double(mm) * nn * std::max(1, kk) * std::max(1, se - sb));
-	};
-	for (const Entry& e : ents) {
-		const int64_t mn   = int64_t(e.m) * e.n;
-		const bool    mult = e.k > 0 && !alpha_zero;
-		// op(A)^T is staged (k x m): transposed unless op(A) already transposes; op(B) (k x n)
-		// as it is. Conjugation negates the imaginary part.
-		const int fa = (ta ? 0 : VB_TRANS) | cx;
-		const int fb = (tb ? VB_TRANS : 0) | cx;
-		if (!cplx) {
-			int64_t ao = 0, bo = 0;
-			if (mult) {
-				ao = wsz;
-				wsz += stage(copies, e.a, e.lda, e.k, e.m, wsz, fa);
-				bo = wsz;
-				wsz += stage(copies, e.b, e.ldb, e.k, e.n, wsz, fb);
-			}
-			const int sb = int(segs.size());
-			if (mult)
-				seg(bo, ao, e.k);
-			task(csz, e.m, e.n, e.k, sb, int(segs.size()));
-			VbOut o{};
-			o.dst    = e.c;
-			o.src_re = csz;
-			o.src_im = -1;
-			o.rows   = e.m;
-			o.ldc    = e.ldc;
-			o.cplx   = 0;
-			for (int64_t s = 0; s < mn; s += kChunk) {
-				o.start = s;
-				o.len   = std::min(kChunk, mn - s);
-				outs.push_back(o);
-			}
-			csz += mn;
-		} else {
-			// Ar, Ai, -Ai (as op(A)^T, k x m), then Br, Bi (k x n); conj of A or B flips the
-			// imaginary sign.
-			const int na = (ta == 2) ? VB_NEG : 0;
-			const int nb = (tb == 2) ? VB_NEG : 0;
-			int64_t   ar = 0, ai = 0, nai = 0, br = 0, bi = 0;
-			if (mult) {
-				ar = wsz;
-				wsz += stage(copies, e.a, e.lda, e.k, e.m, wsz, fa);
-				ai = wsz;
-				wsz += stage(copies, e.a, e.lda, e.k, e.m, wsz, fa | VB_IMAG | na);
-				nai = wsz;
-				wsz += stage(copies, e.a, e.lda, e.k, e.m, wsz, fa | VB_IMAG | (na ^ VB_NEG));
-				br = wsz;
-				wsz += stage(copies, e.b, e.ldb, e.k, e.n, wsz, fb);
-				bi = wsz;
-				wsz += stage(copies, e.b, e.ldb, e.k, e.n, wsz, fb | VB_IMAG | nb);
-			}
-			const int64_t cr = csz, ci = csz + mn;
-			int           sb = int(segs.size());
-			if (mult) {
-				seg(br, ar, e.k);
-				seg(bi, nai, e.k);
-			}
-			task(cr, e.m, e.n, e.k, sb, int(segs.size()));
-			sb = int(segs.size());
-			if (mult) {
-				seg(bi, ar, e.k);
-				seg(br, ai, e.k);
-			}
-			task(ci, e.m, e.n, e.k, sb, int(segs.size()));
-			VbOut o{};
-			o.dst    = e.c;
-			o.src_re = cr;
-			o.src_im = ci;
-			o.rows   = e.m;
-			o.ldc    = e.ldc;
-			o.cplx   = 1;
-			for (int64_t s = 0; s < mn; s += kChunk) {
-				o.start = s;
-				o.len   = std::min(kChunk, mn - s);
-				outs.push_back(o);
-			}
-			csz += 2 * mn;
-		}
-	}
-	// 64 x 64 output tiles, largest tasks first.
-	std::vector<int> order(tasks.size());
-	std::iota(order.begin(), order.end(), 0);
-	std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return cost[size_t(x)] > cost[size_t(y)]; });
-	std::vector<Tile> tiles;
-	for (int t : order)
-		for (int m0 = 0; m0 < std::max(tasks[size_t(t)].m, 1); m0 += 64)
-			for (int n0 = 0; n0 < std::max(tasks[size_t(t)].n, 1); n0 += 64)
-				tiles.push_back(Tile{ t, m0, n0, 0 });
-	if (tiles.size() > size_t(0x7fffffff) || copies.size() > size_t(0x7fffffff)
-	    || outs.size() > size_t(0x7fffffff))
-		throw std::runtime_error("gemm_vbatch: batch too large for one launch");
-	for (const PSeg& s : segs)
-		if (!panel_ld_fits(s.ldl) || !panel_ld_fits(s.ldr))
+	for (const VbEntry& e : ents)
+		if (!panel_ld_fits(panel_ld(e.k)))
 			throw std::runtime_error("gemm_vbatch: a contraction is too long for the panel kernel");
+	VbLaunch p {};
+	p.cplx      = cplx;
+	p.ta        = ta;
+	p.tb        = tb;
+	p.ar        = alpha[0];
+	p.ai        = cplx ? alpha[1] : 0.0;
+	p.br        = beta[0];
+	p.bi        = cplx ? beta[1] : 0.0;
+	p.beta_zero = p.br == 0.0 && p.bi == 0.0;
+	// 64 x 64 tiles from four per CU on (half the LDS and operand traffic per product); below, four
+	// times as many 32 x 32 ones balance better. Two calls of a transformation step with 32- / 64-wide
+	// tiles: m = 2048 (443 and 830 tiles of 64 x 64) 187 / 210 us, m = 4096 (1700 and 3200)
+	// 951 / 814 us, m = 6000 2720 / 2177 us.
+	double tiles64 = 0;
+	for (const VbEntry& e : ents) {
+		tiles64 += double((e.m + 63) / 64) * double((e.n + 63) / 64);
+		p.wide = p.wide || e.lda > kVbNarrowLd || e.ldb > kVbNarrowLd;
+	}
+	p.tile = tiles64 < 4 * 256 ? 32 : 64;
+	if (tiles64 * double(64 / p.tile) * double(64 / p.tile) > double(0x7fffffff / kXcds))
+		throw std::runtime_error("gemm_vbatch: batch too large for one launch");
+	const RunLists lists   = list_runs(ents, p.tile);
+	const size_t   scalar  = (cplx ? 2 : 1) * sizeof(double);
+	const bool     through = outputs_meet_inputs(ents, ta, tb, scalar);
 
-	std::vector<void*> owned;
+	const size_t ebytes = ents.size() * sizeof(VbEntry), rbytes = lists.runs.size() * sizeof(VbRun);
+	void*        host = nullptr;
+	void*        dev  = nullptr;
+	void*        work = nullptr;
+	hipStream_t  s    = nullptr;
+	auto         give_back = [&] {
+                pool_host_free(host);
+                pool_device_free(dev);
+                pool_device_free(work);
+	};
 	try {
-		double* ws = static_cast<double*>(pool_device_alloc(size_t(std::max<int64_t>(wsz, 1)) * sizeof(double)));
-		owned.push_back(ws);
-		double* cw = static_cast<double*>(pool_device_alloc(size_t(std::max<int64_t>(csz, 1)) * sizeof(double)));
-		owned.push_back(cw);
-		VbCopy* d_copies = upload(copies, owned);
-		VbOut*  d_outs   = upload(outs, owned);
-		PTask*  d_tasks  = upload(tasks, owned);
-		PSeg*   d_segs   = upload(segs, owned);
-		Tile*   d_tiles  = upload(tiles, owned);
-		hipStream_t s = nullptr;
-		launch_vb_copy(d_copies, int(copies.size()), ws, s);
-		const double*  bases[PBASE_COUNT] = { ws, ws, ws, ws, ws };
-		const PStrides vs { 0, 0, 0 };
-		launch_panel_gemm<double, double>(64, 64, 0, 2, 1, d_tasks, d_segs, d_tiles,
-		                                  int(tiles.size()), bases, vs, cw, 0, nullptr, 0, 1, 0, s);
-		DMK_HIP_CHECK(hipGetLastError());
-		launch_vb_scatter(d_outs, int(outs.size()), cw, alpha[0], cplx ? alpha[1] : 0.0, beta[0],
-		                  cplx ? beta[1] : 0.0, beta_zero ? 1 : 0, s);
+		if (through) {
+			size_t elems = 0;
+			for (const VbEntry& e : ents)
+				elems += size_t(e.m) * size_t(e.n);
+			work = pool_device_alloc(elems * scalar);
+			double* at = static_cast<double*>(work);
+			for (VbEntry& e : ents) {
+				e.d   = at;
+				e.ldd = e.m;
+				at += size_t(e.m) * size_t(e.n) * (cplx ? 2 : 1);
+			}
+		}
+		host = pool_host_alloc(ebytes + rbytes);
+		dev  = pool_device_alloc(ebytes + rbytes);
+		std::memcpy(host, ents.data(), ebytes);
+		std::memcpy(static_cast<char*>(host) + ebytes, lists.runs.data(), rbytes);
+		DMK_HIP_CHECK(hipMemcpyAsync(dev, host, ebytes + rbytes, hipMemcpyHostToDevice, s));
+		const VbEntry* d_ents = static_cast<const VbEntry*>(dev);
+		const VbRun*   d_runs = reinterpret_cast<const VbRun*>(static_cast<char*>(dev) + ebytes);
+		launch_vb_gemm(p, d_ents, d_runs, lists.nruns, int(lists.longest), s);
+		if (through)
+			launch_vb_copy_back(d_ents, int(ents.size()), cplx, s);
 		DMK_HIP_CHECK(hipStreamSynchronize(s));
 	} catch (...) {
 		(void)hipDeviceSynchronize();
-		for (void* p : owned)
-			pool_device_free(p);
+		give_back();
 		throw;
 	}
-	for (void* p : owned)
-		pool_device_free(p);
+	give_back();
 }
 
 } // namespace dmk

@@ -1,5 +1,5 @@
 // Variable-size batched GEMM over caller pointers (the dmrg_Xgemm_vbatch boundary of the
-// reference plugin, GPUPlugin/dmrg_vbatch.cpp:129-652), built on the K-major panel kernel.
+// reference plugin, GPUPlugin/dmrg_vbatch.cpp:129-652).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -9,46 +9,45 @@
 
 namespace dmk {
 
-enum VbFlags : int32_t
-{
-	VB_TRANS = 1, // destination (i, j) = source (j, i)
-	VB_CPLX  = 2, // source is interleaved complex
-	VB_IMAG  = 4, // take the imaginary part (else the real part)
-	VB_NEG   = 8, // negate
+// One product D = alpha op(A) op(B) + beta C (column major; complex scalars interleaved, leading
+// dimensions in scalars). D is C, or a workspace where C overlaps an operand.
+struct VbEntry {
+	const double* a;
+	const double* b;
+	const double* c;
+	double*       d;
+	int32_t       m, n, k;
+	int32_t       lda, ldb, ldc, ldd;
+	int32_t       pad;
 };
 
-// One chunk [start, start + len) of a column-major destination matrix (rows x ?, leading
-// dimension ldd >= rows, zeros in rows [rows, ldd)) at element offset dst of the staging
-// workspace, read from src with leading dimension ld.
-struct VbCopy {
-	const double* src;
-	int64_t       dst;
-	int64_t       start;
-	int64_t       len;
-	int32_t       rows;
-	int32_t       ld;
-	int32_t       flags;
-	int32_t       ldd;
+// Output tiles [t0, t1) of an entry (column major over its tile grid), which sit at positions
+// first, first + 1, ... of one XCD's list.
+struct VbRun {
+	int32_t first;
+	int32_t entry;
+	int32_t t0;
+	int32_t t1;
 };
 
-// One chunk of a result scattered into the caller's C (rows x ?, leading dimension ldc):
-// C = alpha * W + beta * C with W the compact workspace result (real part at src_re, imaginary
-// part at src_im for complex).
-struct VbOut {
-	double* dst;
-	int64_t src_re;
-	int64_t src_im;
-	int64_t start;
-	int64_t len;
-	int32_t rows;
-	int32_t ldc;
-	int32_t cplx;
-	int32_t pad;
+struct VbLaunch {
+	bool   cplx;
+	int    ta, tb;   // 0 N, 1 T, 2 C
+	int    tile;     // 32 or 64
+	bool   wide;     // 64-bit operand offsets (leading dimensions past kVbNarrowLd)
+	double ar, ai, br, bi;
+	bool   beta_zero;
 };
 
-void launch_vb_copy(const VbCopy* jobs, int njobs, double* ws, hipStream_t s);
-void launch_vb_scatter(const VbOut* jobs, int njobs, const double* cw, double ar, double ai,
-                       double br, double bi, int beta_zero, hipStream_t s);
+// Largest leading dimension whose byte offsets within a tile fit 32 bits (64 rows, 16 bytes).
+constexpr int kVbNarrowLd = 1 << 21;
+
+// runs: eight lists of nruns each, by position (filled up with first = INT32_MAX); `longest`
+// positions in the longest list.
+void launch_vb_gemm(const VbLaunch& p, const VbEntry* entries, const VbRun* runs, int nruns,
+                    int longest, hipStream_t s);
+// C = D for every entry (the workspace results of overlapping batches).
+void launch_vb_copy_back(const VbEntry* entries, int nentries, bool cplx, hipStream_t s);
 
 // C_e = alpha op(A_e) op(B_e) + beta C_e for every entry e of every group (m, n, k, lda, ldb,
 // ldc per group; pointers per entry, device memory, expanded in group order). cplx selects

@@ -92,3 +92,53 @@ def test_gpu_vbatch_alpha_zero_scales_c_only():
     dm.gemm_vbatch("N", "N", [(m, n, k, m, k, m, [(dA.ptr, dA.ptr, dC.ptr)])], alpha=0.0,
                    beta=3.0)
     np.testing.assert_array_equal(dC.download().reshape(m, n, order="F"), 3.0 * C)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("cplx", [False, True])
+@pytest.mark.parametrize("transa,transb", [("N", "N"), ("N", "T"), ("T", "N"), ("T", "T")])
+def test_gpu_vbatch_large_batch_tiles(transa, transb, cplx):
+    # Enough tiles for the 64 x 64 kernel (2048 of them), k at every remainder of a 16-element chunk
+    # and past the three chunks in flight, an odd base address; a few leading dimensions past the
+    # 32-bit offsets select the other variant.
+    rng = np.random.default_rng(3)
+    w = 2 if cplx else 1
+    dt = np.complex128 if cplx else np.float64
+    tall = 64 * 64
+    shapes = [(tall, 64 * 33, 17), (129, 63, 15), (33, 65, 16), (64, 64, 47), (31, 97, 64), (1, 1, 100)]
+    buf = rng.uniform(-1, 1, w * (tall * 128 + 1))
+    dX = dm.DeviceArray.from_host(buf)
+    view = buf[1:1 + w * tall * 128].view(dt)
+    groups, outs = [], []
+    for m, n, k in shapes:
+        lda, ldb = (k if transa != "N" else m) + 1, (n if transb != "N" else k) + 2
+        A = view[:lda * (m if transa != "N" else k)].reshape((lda, -1), order="F")[:lda - 1]
+        B = view[:ldb * (k if transb != "N" else n)].reshape((ldb, -1), order="F")[:ldb - 2]
+        dC = dm.DeviceArray(w * m * n)
+        groups.append((m, n, k, lda, ldb, m, [(dX.ptr + 8, dX.ptr + 8, dC.ptr)]))
+        outs.append((dC, _op(A, transa) @ _op(B, transb)))
+    dm.gemm_vbatch(transa, transb, groups, cplx=cplx)
+    for (dC, want), (m, n, k) in zip(outs, shapes):
+        got = dC.download().view(dt).reshape((m, n), order="F")
+        # k products of at most 1 (2 for complex), k + 2 roundings each way.
+        assert np.abs(got - want).max() <= 2 * w * w * k * (k + 2) * 2.0 ** -53
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("wide", [False, True])
+def test_gpu_vbatch_output_over_input_and_wide_rows(wide):
+    # C in the memory of A (computed through a workspace), and a leading dimension past 2^21.
+    rng = np.random.default_rng(4)
+    m, n, k = 5, 3, 4
+    ld = (1 << 21) + 3 if wide else m
+    X = rng.uniform(-1, 1, ld * 4)
+    B = rng.uniform(-1, 1, (k, n))
+    dX, dB = dm.DeviceArray.from_host(X), dm.DeviceArray.from_host(B.ravel(order="F"))
+    A = X.reshape((ld, 4), order="F")[:m, :k].copy()
+    dm.gemm_vbatch("N", "N", [(m, n, k, ld, k, ld, [(dX.ptr, dB.ptr, dX.ptr)])], alpha=2.0, beta=0.5)
+    got = dX.download().reshape((ld, 4), order="F")
+    want = 2.0 * A @ B + 0.5 * A[:, :n]
+    assert np.abs(got[:m, :n] - want).max() <= 16 * (k + 3) * 2.0 ** -53
+    np.testing.assert_array_equal(got[:m, n:], A[:, n:])
+    if wide:
+        np.testing.assert_array_equal(got[m:], X.reshape((ld, 4), order="F")[m:])
