@@ -18,6 +18,7 @@
 
 #include <chrono>
 #include <cmath>
+#include <cstdint>
 #include <stdexcept>
 #include <string>
 
@@ -36,15 +37,13 @@ void launch_combine(double* z, const double* V, int64_t ld, const double* c, int
                     hipStream_t s);
 void launch_residual(const double* hx, const double* x, double e, int64_t n, double* partial,
                      double* out, hipStream_t s);
-void launch_dot_at(const double* x, const double* y, int64_t n, double* partial, double* base,
-                   const int* jdev, int offset, hipStream_t s);
-void launch_lanczos_update_at(double* v2, const double* v1, const double* v0, const double* A,
-                              const double* B, const int* jdev, int64_t n, double* partial,
-                              double* norm_out, hipStream_t s);
-void launch_finish_step(double* v2, double* basis, int64_t n, const double* nrm, const int* jdev,
-                        hipStream_t s);
-void launch_step_scalars(const double* A, double* B, const double* nrm, int* jdev, int maxn,
-                         double* report, hipStream_t s);
+void launch_dot_step(const double* x, const double* y, int64_t n, double* partial, int* jdev,
+                     hipStream_t s);
+void launch_lanczos_update_step(double* v2, const double* v1, const double* v0, double* A,
+                                const double* B, const int* jdev, int64_t n, const double* pdot,
+                                double* pnorm, hipStream_t s);
+void launch_finish_step(double* v2, double* basis, int64_t n, const double* pnorm, const double* A,
+                        double* B, const int* jdev, int maxn, double* host, hipStream_t s);
 void launch_copy(double* y, const double* x, int64_t n, hipStream_t s);
 
 LanczosWorkspace::~LanczosWorkspace()
@@ -77,7 +76,7 @@ void LanczosWorkspace::reserve(int64_t n, int columns)
 	cols_ = 0;
 	auto dev = [](size_t bytes) { return static_cast<double*>(pool_device_alloc(bytes)); };
 	basis_   = dev(size_t(n) * size_t(columns) * sizeof(double));
-	partial_ = dev(size_t(reduction_blocks()) * sizeof(double));
+	partial_ = dev(2 * size_t(reduction_blocks()) * sizeof(double)); // dot, norm
 	scal_    = dev(size_t(3 * columns + 8) * sizeof(double));
 	tmp_     = dev(size_t(n) * sizeof(double));
 	tmp2_    = dev(size_t(n) * sizeof(double));
@@ -113,6 +112,45 @@ struct StepGraphs {
 		}
 	}
 };
+
+// The step report in pinned memory (alpha_j, beta_{j+1}), polled for instead of waiting for the
+// stream: a stream wait and the next launch after it left the chip idle for 35 to 50 us per step.
+// Cleared to a bit pattern no computation gives; the kernel stores both values whole.
+constexpr uint64_t kNoReport = ~uint64_t(0);
+
+void clear_report(double* report)
+{
+	for (int i = 0; i < 2; ++i)
+		__atomic_store_n(reinterpret_cast<uint64_t*>(report) + i, kNoReport, __ATOMIC_RELEASE);
+}
+
+// Returns once both values are there. Ends also when the stream has finished (then they are, or
+// its work failed) or reports an error, looked up every 50 us.
+void wait_report(double* report, hipStream_t s)
+{
+	auto there = [&] {
+		const uint64_t* r = reinterpret_cast<const uint64_t*>(report);
+		return __atomic_load_n(r, __ATOMIC_ACQUIRE) != kNoReport
+		       && __atomic_load_n(r + 1, __ATOMIC_ACQUIRE) != kNoReport;
+	};
+	using clock = std::chrono::steady_clock;
+	auto look   = clock::now() + std::chrono::microseconds(50);
+	while (!there()) {
+		if (clock::now() < look)
+			continue;
+		const hipError_t e = hipStreamQuery(s);
+		if (e == hipSuccess)
+			break;
+		if (e != hipErrorNotReady)
+			DMK_HIP_CHECK(e);
+		look = clock::now() + std::chrono::microseconds(50);
+	}
+	if (!there()) {
+		DMK_HIP_CHECK(hipStreamSynchronize(s));
+		if (!there())
+			throw std::runtime_error("lanczos: a step ended without its report");
+	}
+}
 
 // noise: relative matvec noise of a reduced-precision run that an FP64 restart follows (0 for
 // a plain run); see noise_reached below.
@@ -157,19 +195,27 @@ Decomp decompose(Plan& plan, LanczosWorkspace& ws, const double* init, int max_s
 	launch_scale_copy(ws.basis(0), init, NRM + 1, n, s);
 
 	// First step (LanczosCore.h:181-208): V1 = H V0, alpha_0, V1 -= alpha_0 V0, beta_1, V1 /= beta_1.
-	matvec(ws.basis(0), ws.basis(1));
+	// Enqueued without waiting: the step graphs are captured while it runs.
+	DMK_HIP_CHECK(hipEventRecord(ev0, s));
+	plan.apply(ws.basis(0), n, ws.basis(1), n, 1, 0);
+	DMK_HIP_CHECK(hipEventRecord(ev1, s));
 	d.matvecs++;
 	launch_dot(ws.basis(0), ws.basis(1), n, part, A, 0, s);
 	launch_lanczos_update(ws.basis(1), ws.basis(0), ws.basis(0), A, B, n, part, NRM, s);
 	launch_scale(ws.basis(1), NRM + 1, n, s);
 	DMK_HIP_CHECK(hipMemcpyAsync(host, A, sizeof(double), hipMemcpyDeviceToHost, s));
 	DMK_HIP_CHECK(hipMemcpyAsync(host + 1, NRM, sizeof(double), hipMemcpyDeviceToHost, s));
-	DMK_HIP_CHECK(hipStreamSynchronize(s));
-	d.a[0] = host[0];
-	if (maxn > 1) {
-		d.b[1] = host[1];
+	if (maxn > 1)
 		DMK_HIP_CHECK(hipMemcpyAsync(B + 1, NRM, sizeof(double), hipMemcpyDeviceToDevice, s));
-	}
+	auto first_step_done = [&] {
+		DMK_HIP_CHECK(hipStreamSynchronize(s));
+		float ms = 0;
+		DMK_HIP_CHECK(hipEventElapsedTime(&ms, ev0, ev1));
+		ms_matvec += ms;
+		d.a[0] = host[0];
+		if (maxn > 1)
+			d.b[1] = host[1];
+	};
 
 	double eold  = 0;
 	int    j     = 1;
@@ -196,12 +242,12 @@ Decomp decompose(Plan& plan, LanczosWorkspace& ws, const double* init, int max_s
 	if (use_graph && !reortho && maxn > 1) {
 		// Ring of three fixed vectors: V_{j-1}, V_j, V_{j+1} live in ring[(j-1)%3], ring[j%3],
 		// ring[(j+1)%3]; each captured step also writes V_{j+1} to basis column j+1.
-		double* report = ws.scal() + 3 * cap + 4;
+		double* pnorm = part + reduction_blocks();
 		launch_copy(ws.ring(0), ws.basis(0), n, s);
 		launch_copy(ws.ring(1), ws.basis(1), n, s);
-		const int one = 1;
-		DMK_HIP_CHECK(hipMemcpyAsync(ws.jdev(), &one, sizeof(int), hipMemcpyHostToDevice, s));
-		DMK_HIP_CHECK(hipStreamSynchronize(s));
+		DMK_HIP_CHECK(hipMemsetAsync(ws.jdev(), 0, sizeof(int), s)); // before the first captured step
+		// The captured steps report into host[2], host[3]; host[0], host[1] are the first step's.
+		double*    report = host + 2;
 		StepGraphs sg;
 		for (int p = 0; p < 3; ++p) {
 			double* v0 = ws.ring((p + 2) % 3);
@@ -214,13 +260,10 @@ Decomp decompose(Plan& plan, LanczosWorkspace& ws, const double* init, int max_s
 			hipError_t ec = hipSuccess;
 			try {
 				plan.apply(v1, n, v2, n, 1, 0);
-				launch_dot_at(v1, v2, n, part, A, ws.jdev(), 0, s);
-				launch_lanczos_update_at(v2, v1, v0, A, B, ws.jdev(), n, part, NRM, s);
-				launch_finish_step(v2, ws.basis(0), n, NRM, ws.jdev(), s);
-				launch_step_scalars(A, B, NRM, ws.jdev(), maxn, report, s);
+				launch_dot_step(v1, v2, n, part, ws.jdev(), s);
+				launch_lanczos_update_step(v2, v1, v0, A, B, ws.jdev(), n, part, pnorm, s);
+				launch_finish_step(v2, ws.basis(0), n, pnorm, A, B, ws.jdev(), maxn, report, s);
 				ec = hipGetLastError();
-				if (ec == hipSuccess)
-					ec = hipMemcpyAsync(host, report, 2 * sizeof(double), hipMemcpyDeviceToHost, s);
 			} catch (...) {
 				hipGraph_t partial = nullptr;
 				(void)hipStreamEndCapture(s, &partial);
@@ -235,14 +278,16 @@ Decomp decompose(Plan& plan, LanczosWorkspace& ws, const double* init, int max_s
 				throw std::runtime_error("lanczos: stream capture produced no graph");
 			DMK_HIP_CHECK(hipGraphInstantiate(&sg.e[p], sg.g[p], nullptr, nullptr, 0));
 		}
+		first_step_done();
 		const auto t0 = std::chrono::steady_clock::now();
 		for (j = 1; j < maxn; ++j) {
+			clear_report(report);
 			DMK_HIP_CHECK(hipGraphLaunch(sg.e[j % 3], s));
-			DMK_HIP_CHECK(hipStreamSynchronize(s));
+			wait_report(report, s);
 			d.matvecs++;
-			d.a[size_t(j)] = host[0];
+			d.a[size_t(j)] = report[0];
 			if (j + 1 < maxn)
-				d.b[size_t(j + 1)] = host[1];
+				d.b[size_t(j + 1)] = report[1];
 			const double e     = tridiag_eigenvalue(d.a.data(), d.b.data(), j + 1, 0);
 			const double delta = std::fabs(e - eold);
 			eold               = e;
@@ -254,47 +299,49 @@ Decomp decompose(Plan& plan, LanczosWorkspace& ws, const double* init, int max_s
 		}
 		// Device time is not split out per matvec inside the graphs; charge the loop.
 		ms_matvec += std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
-	} else
-	for (j = 1; j < maxn; ++j) {
-		double* v0 = ws.basis(j - 1);
-		double* v1 = ws.basis(j);
-		double* v2 = ws.basis(j + 1);
-		// oneStepDecomposition (LanczosVectors.h:203-237).
-		matvec(v1, v2);
-		d.matvecs++;
-		launch_dot(v1, v2, n, part, A + j, 0, s);
-		launch_lanczos_update(v2, v1, v0, A + j, B + j, n, part, NRM, s);
-		launch_scale(v2, NRM + 1, n, s);
-		DMK_HIP_CHECK(hipMemcpyAsync(host, A + j, sizeof(double), hipMemcpyDeviceToHost, s));
-		DMK_HIP_CHECK(hipMemcpyAsync(host + 1, NRM, sizeof(double), hipMemcpyDeviceToHost, s));
-		if (j + 1 < maxn)
-			DMK_HIP_CHECK(hipMemcpyAsync(B + j + 1, NRM, sizeof(double), hipMemcpyDeviceToDevice, s));
-		if (reortho) {
-			// reorthoIfNecessary (LanczosVectors.h:243-271): V2 -= <V_i|V2> V_i for i = 0..j in turn,
-			// then renormalize.
-			for (int i = 0; i <= j; ++i) {
-				launch_dot(ws.basis(i), v2, n, part, DOT, 0, s);
-				launch_axpy_neg(v2, ws.basis(i), DOT, n, s);
+	} else {
+		first_step_done();
+		for (j = 1; j < maxn; ++j) {
+			double* v0 = ws.basis(j - 1);
+			double* v1 = ws.basis(j);
+			double* v2 = ws.basis(j + 1);
+			// oneStepDecomposition (LanczosVectors.h:203-237).
+			matvec(v1, v2);
+			d.matvecs++;
+			launch_dot(v1, v2, n, part, A + j, 0, s);
+			launch_lanczos_update(v2, v1, v0, A + j, B + j, n, part, NRM, s);
+			launch_scale(v2, NRM + 1, n, s);
+			DMK_HIP_CHECK(hipMemcpyAsync(host, A + j, sizeof(double), hipMemcpyDeviceToHost, s));
+			DMK_HIP_CHECK(hipMemcpyAsync(host + 1, NRM, sizeof(double), hipMemcpyDeviceToHost, s));
+			if (j + 1 < maxn)
+				DMK_HIP_CHECK(hipMemcpyAsync(B + j + 1, NRM, sizeof(double), hipMemcpyDeviceToDevice, s));
+			if (reortho) {
+				// reorthoIfNecessary (LanczosVectors.h:243-271): V2 -= <V_i|V2> V_i for i = 0..j in turn,
+				// then renormalize.
+				for (int i = 0; i <= j; ++i) {
+					launch_dot(ws.basis(i), v2, n, part, DOT, 0, s);
+					launch_axpy_neg(v2, ws.basis(i), DOT, n, s);
+				}
+				launch_dot(v2, v2, n, part, DOT, 2, s);
+				launch_scale(v2, DOT + 1, n, s);
 			}
-			launch_dot(v2, v2, n, part, DOT, 2, s);
-			launch_scale(v2, DOT + 1, n, s);
-		}
-		DMK_HIP_CHECK(hipStreamSynchronize(s));
-		d.a[size_t(j)] = host[0];
-		if (j + 1 < maxn)
-			d.b[size_t(j + 1)] = host[1];
-		// ab.diag(tmpEigs, j+1) and the stop test (LanczosCore.h:220-240).
-		const double e     = tridiag_eigenvalue(d.a.data(), d.b.data(), j + 1, 0);
-		const double delta = std::fabs(e - eold);
-		eold               = e;
-		bool exitFlag      = (delta < tol) || (j == maxn - 1) || noise_reached(j, e);
-		if (exitFlag && n <= 4) {
-			broke = true;
-			break;
-		}
-		if (exitFlag && j >= min_steps) {
-			broke = true;
-			break;
+			DMK_HIP_CHECK(hipStreamSynchronize(s));
+			d.a[size_t(j)] = host[0];
+			if (j + 1 < maxn)
+				d.b[size_t(j + 1)] = host[1];
+			// ab.diag(tmpEigs, j+1) and the stop test (LanczosCore.h:220-240).
+			const double e     = tridiag_eigenvalue(d.a.data(), d.b.data(), j + 1, 0);
+			const double delta = std::fabs(e - eold);
+			eold               = e;
+			bool exitFlag      = (delta < tol) || (j == maxn - 1) || noise_reached(j, e);
+			if (exitFlag && n <= 4) {
+				broke = true;
+				break;
+			}
+			if (exitFlag && j >= min_steps) {
+				broke = true;
+				break;
+			}
 		}
 	}
 	d.m = (broke || j < maxn) ? j + 1 : maxn;

@@ -8,6 +8,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 namespace dmk {
 
 constexpr int kRedBlocks  = 1024;
@@ -167,28 +169,52 @@ __global__ void copy_kernel(double* __restrict__ y, const double* __restrict__ x
 // Step-indexed kernels of the captured Lanczos step: the current step j is read from device
 // memory (jdev), so one captured graph serves every step of its ring phase.
 
-// base[*jdev + offset] = sum(partial[0..np)).
-__global__ __launch_bounds__(kRedThreads) void reduce_final_at_kernel(const double* __restrict__ partial,
-                                                                      int np, double* __restrict__ base,
-                                                                      const int* __restrict__ jdev,
-                                                                      int offset)
+// The kernels of one captured Lanczos step: three launches, each reduction finished by the kernel
+// that needs its result. Every workgroup sums the kRedBlocks partials again, in the order of
+// reduce_final_kernel (8 KB from L2), instead of waiting for a launch of one workgroup to do so;
+// the step's scalars are written by the workgroup that has them, and the host reads alpha_j and
+// beta_{j+1} from pinned memory. Seven dependent launches and copies of 4 to 6 us each took 43 us
+// per step beside the matvec at n = 7e5; three take 16 us, without gaps in the captured graph.
+
+// Sum of the partials, in every thread of the workgroup.
+__device__ inline double partials_sum(const double* __restrict__ partial, int np)
 {
-	double s = 0;
+	__shared__ double total;
+	double            s = 0;
 	for (int i = threadIdx.x; i < np; i += blockDim.x)
 		s += partial[i];
 	s = block_sum(s);
 	if (threadIdx.x == 0)
-		base[*jdev + offset] = s;
+		total = s;
+	__syncthreads();
+	return total;
 }
 
-// v2 = v2 - A[j] v1 - B[j] v0, partial sums of |v2|^2.
-__global__ __launch_bounds__(kRedThreads) void lanczos_update_at_kernel(
+// Partials of x . y; *jdev becomes this step's index.
+__global__ __launch_bounds__(kRedThreads) void dot_step_kernel(const double* __restrict__ x,
+                                                               const double* __restrict__ y,
+                                                               int64_t n, double* __restrict__ partial,
+                                                               int* __restrict__ jdev)
+{
+	double  s      = 0;
+	int64_t stride = int64_t(gridDim.x) * blockDim.x;
+	for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += stride)
+		s += x[i] * y[i];
+	s = block_sum(s);
+	if (threadIdx.x == 0)
+		partial[blockIdx.x] = s;
+	if (threadIdx.x == 0 && blockIdx.x == 0)
+		*jdev += 1;
+}
+
+// A[j] = alpha (the sum of pdot), v2 -= alpha v1 + B[j] v0, partials of |v2|^2 into pnorm.
+__global__ __launch_bounds__(kRedThreads) void lanczos_update_step_kernel(
     double* __restrict__ v2, const double* __restrict__ v1, const double* __restrict__ v0,
-    const double* __restrict__ A, const double* __restrict__ B, const int* __restrict__ jdev,
-    int64_t n, double* __restrict__ partial)
+    double* __restrict__ A, const double* __restrict__ B, const int* __restrict__ jdev, int64_t n,
+    const double* __restrict__ pdot, double* __restrict__ pnorm)
 {
 	const int    j      = *jdev;
-	const double a      = A[j];
+	const double a      = partials_sum(pdot, kRedBlocks);
 	const double b      = B[j];
 	double       s      = 0;
 	int64_t      stride = int64_t(gridDim.x) * blockDim.x;
@@ -199,39 +225,36 @@ __global__ __launch_bounds__(kRedThreads) void lanczos_update_at_kernel(
 	}
 	s = block_sum(s);
 	if (threadIdx.x == 0)
-		partial[blockIdx.x] = s;
+		pnorm[blockIdx.x] = s;
+	if (threadIdx.x == 0 && blockIdx.x == 0)
+		A[j] = a;
 }
 
-// v2 *= nrm[1] and basis column j+1 = v2.
-__global__ void finish_step_kernel(double* __restrict__ v2, double* __restrict__ basis, int64_t n,
-                                   const double* __restrict__ nrm, const int* __restrict__ jdev)
+// beta = the root of the sum of pnorm: v2 /= beta, also into basis column j + 1; B[j + 1] = beta
+// (j + 1 < maxn), and (A[j], beta) to the host.
+__global__ __launch_bounds__(kRedThreads) void finish_step_kernel(
+    double* __restrict__ v2, double* __restrict__ basis, int64_t n, const double* __restrict__ pnorm,
+    const double* __restrict__ A, double* __restrict__ B, const int* __restrict__ jdev, int maxn,
+    double* __restrict__ host)
 {
-	const double  inv    = nrm[1];
-	double*       col    = basis + int64_t(*jdev + 1) * n;
+	const int     j      = *jdev;
+	const double  beta   = sqrt(partials_sum(pnorm, kRedBlocks));
+	const double  inv    = (beta > 0) ? 1.0 / beta : 0.0;
+	double*       col    = basis + int64_t(j + 1) * n;
 	int64_t       stride = int64_t(gridDim.x) * blockDim.x;
 	for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += stride) {
 		const double v = v2[i] * inv;
 		v2[i]          = v;
 		col[i]         = v;
 	}
-}
-
-// report = (A[j], |v2|); B[j+1] = |v2| when j+1 < maxn; j += 1.
-__global__ void step_scalars_kernel(const double* __restrict__ A, double* __restrict__ B,
-                                    const double* __restrict__ nrm, int* __restrict__ jdev,
-                                    int maxn, double* __restrict__ report)
-{
 	if (threadIdx.x == 0 && blockIdx.x == 0) {
-		const int j = *jdev;
-		report[0]   = A[j];
-		report[1]   = nrm[0];
 		if (j + 1 < maxn)
-			B[j + 1] = nrm[0];
-		*jdev = j + 1;
+			B[j + 1] = beta;
+		// Seen by the host while the kernel still runs (it polls; see lanczos.cpp).
+		__hip_atomic_store(host, A[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+		__hip_atomic_store(host + 1, beta, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 	}
 }
-
-// Host launchers ------------------------------------------------------------------------------
 
 namespace {
 unsigned grid_for(int64_t n)
@@ -296,36 +319,27 @@ void launch_residual(const double* hx, const double* x, double e, int64_t n, dou
 	                   out, 1);
 }
 
-void launch_dot_at(const double* x, const double* y, int64_t n, double* partial, double* base,
-                   const int* jdev, int offset, hipStream_t s)
+void launch_dot_step(const double* x, const double* y, int64_t n, double* partial, int* jdev,
+                     hipStream_t s)
 {
-	hipLaunchKernelGGL(dot_partial_kernel, dim3(kRedBlocks), dim3(kRedThreads), 0, s, x, y, n,
-	                   partial);
-	hipLaunchKernelGGL(reduce_final_at_kernel, dim3(1), dim3(kRedThreads), 0, s, partial,
-	                   kRedBlocks, base, jdev, offset);
-}
-
-void launch_lanczos_update_at(double* v2, const double* v1, const double* v0, const double* A,
-                              const double* B, const int* jdev, int64_t n, double* partial,
-                              double* norm_out, hipStream_t s)
-{
-	hipLaunchKernelGGL(lanczos_update_at_kernel, dim3(kRedBlocks), dim3(kRedThreads), 0, s, v2, v1,
-	                   v0, A, B, jdev, n, partial);
-	hipLaunchKernelGGL(reduce_final_kernel, dim3(1), dim3(kRedThreads), 0, s, partial, kRedBlocks,
-	                   norm_out, 2);
-}
-
-void launch_finish_step(double* v2, double* basis, int64_t n, const double* nrm, const int* jdev,
-                        hipStream_t s)
-{
-	hipLaunchKernelGGL(finish_step_kernel, dim3(grid_for(n)), dim3(256), 0, s, v2, basis, n, nrm,
+	hipLaunchKernelGGL(dot_step_kernel, dim3(kRedBlocks), dim3(kRedThreads), 0, s, x, y, n, partial,
 	                   jdev);
 }
 
-void launch_step_scalars(const double* A, double* B, const double* nrm, int* jdev, int maxn,
-                         double* report, hipStream_t s)
+void launch_lanczos_update_step(double* v2, const double* v1, const double* v0, double* A,
+                                const double* B, const int* jdev, int64_t n, const double* pdot,
+                                double* pnorm, hipStream_t s)
 {
-	hipLaunchKernelGGL(step_scalars_kernel, dim3(1), dim3(64), 0, s, A, B, nrm, jdev, maxn, report);
+	hipLaunchKernelGGL(lanczos_update_step_kernel, dim3(kRedBlocks), dim3(kRedThreads), 0, s, v2, v1,
+	                   v0, A, B, jdev, n, pdot, pnorm);
+}
+
+void launch_finish_step(double* v2, double* basis, int64_t n, const double* pnorm, const double* A,
+                        double* B, const int* jdev, int maxn, double* host, hipStream_t s)
+{
+	const unsigned grid = std::min(grid_for(n), unsigned(kRedBlocks));
+	hipLaunchKernelGGL(finish_step_kernel, dim3(grid), dim3(kRedThreads), 0, s, v2, basis, n, pnorm,
+	                   A, B, jdev, maxn, host);
 }
 
 void launch_copy(double* y, const double* x, int64_t n, hipStream_t s)
