@@ -843,7 +843,8 @@ Tuning default_tuning(int precision)
 // count, and larger tiles with more residency (two LDS stages) win by less. Timed on Heisenberg
 // and Hubbard superblocks of m = 128 .. 3500 states, all tile shapes x split-k x load depths x
 // K chunks x MFMA forms; matvec in us with 64 x 64 tiles everywhere (the former choice), with the
-// rule, and with the best of all combinations:
+// rule, and with the best of all combinations (the K loop, the result stores and the LDS masks of the
+// kernels have since taken 1 to 5 % off all three; the largest BF16x3 problems have moved to 128 x 128):
 //            t1    t2    FP64                FP32                BF16x3
 //   spin 128   0.1  0.04    40 /   24 /   23    31 /   21 /   21    33 /   28 /   28
 //   spin 512   0.8  0.3     88 /   44 /   42    55 /   33 /   33    58 /   41 /   41
@@ -870,12 +871,16 @@ Tuning Plan::rule_tuning(int precision) const
 		t.kchunk = kchunk;
 	};
 	if (precision == PREC_BF16X3) {
+		// Two waves per SIMD at most: the largest tiles, once they fill the chip, read the least LDS
+		// per MFMA (Hubbard 3072: 128 x 128 tiles 1107 us, 128 x 64 1190).
 		t.mfma32 = t2 < 2.5 ? 1 : 0;
-		t.splitk = t2 < 2.5 ? 2048 : 0;
+		t.splitk = t2 < 2.5 || t2 >= 5 ? 2048 : 0;
 		if (t2 < 2.5)
 			shape(64, 64, 64, 64, 2, 1);
-		else
+		else if (t2 < 5)
 			shape(128, 64, 128, 64, 1, 1);
+		else
+			shape(128, 128, 128, 128, 1, 1);
 		return t;
 	}
 	// FP64 below t2 = 3 keeps the base tuning's order of summation (single K chunks, split-k 2048),

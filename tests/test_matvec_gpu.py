@@ -330,6 +330,42 @@ def test_gpu_balanced_launch_multi_vector(prec):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("size", [97, 700, 1410, 1700, 1900, 2400])
+def test_gpu_rule_shapes(size):
+    # One patch of size x (size + 3) per class of the launch-shape rule (0.02 to 5.6 tiles of
+    # 64 x 64 per CU): every precision against numpy with the modes' usual bounds, several vectors
+    # in one launch bitwise the single vector's, and FP64 below three tiles per CU bitwise the base
+    # tuning's.
+    rng = np.random.default_rng(size)
+    L, R = size, size + 3
+
+    def block(n):
+        return np.asfortranarray(rng.uniform(-1, 1, (n, n)))
+    blocks = {(0, 0, 0): (block(L), np.asfortranarray(np.eye(R))), (0, 0, 1): (block(L), block(R)),
+              (0, 0, 2): (block(L), block(R))}
+    prob = dm.KronProblem(L=[L], R=[R], nC=3, blocks=blocks)
+    n, nvec = prob.n, 3
+    X = rng.uniform(-1, 1, nvec * n)
+    want = prob.apply_numpy(X[:n])
+    dX, dY, dy = dm.DeviceArray.from_host(X), dm.DeviceArray(nvec * n), dm.DeviceArray(n)
+    for prec, tol in (("fp64", 1e-12), ("fp32", 1e-5), ("bf16x3", 1e-4)):
+        op = dm.BatchedGemm(prob, prec)
+        op.apply_Htarget(dX, dy)
+        op.sync()
+        one = dy.download()
+        assert rel_err(one, want) < tol, prec
+        op.apply_multi(dX, dY, nvec)
+        op.sync()
+        assert np.array_equal(dY.download(n), one), prec
+        if prec == "fp64" and size <= 1700:
+            op.set_tuning(**op.tuning())
+            op.apply_Htarget(dX, dy)
+            op.sync()
+            assert np.array_equal(dy.download(), one)
+        op.close()
+
+
+@pytest.mark.gpu
 def test_gpu_autotune_keeps_results():
     left = {-2: 90, 0: 150, 2: 90}
     prob = problems.qn_problem(left, left, 0, problems.heisenberg_links(3), seed=9)
