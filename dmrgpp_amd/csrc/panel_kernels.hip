@@ -514,7 +514,7 @@ __global__ __launch_bounds__(kPThreads) void panel_gemm_kernel(
 					barrier_no_fence();
 					// One exit only: with a second one out of the middle of the loop the compiler
 					// kept the accumulators in two register sets and copied them, behind a wait
-					// for the last MFMA, in every round.
+					// for the last MFMA, every two chunks.
 					if (c + 2 < nch)
 						issue(A0, B0);
 					compute(A1, B1);
