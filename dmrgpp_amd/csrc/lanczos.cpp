@@ -10,6 +10,7 @@
 // is followed by an FP64 restart from the first run's Ritz vector, which converges in a few
 // FP64 matvecs because that vector is already close to the FP64 eigenvector.
 #include "lanczos.h"
+#include "lanczos_step.h"
 
 #include "davidson.h"
 
@@ -96,23 +97,6 @@ struct Decomp {
 	double              energy  = 0;
 };
 
-// One Lanczos decomposition from init (any norm) with the plan's current precision. Leaves the
-// kept vectors in ws.basis(0..m).
-// The three captured phase graphs of one decomposition (ring roles rotate with period 3).
-struct StepGraphs {
-	hipGraph_t     g[3] = { nullptr, nullptr, nullptr };
-	hipGraphExec_t e[3] = { nullptr, nullptr, nullptr };
-	~StepGraphs()
-	{
-		for (int i = 0; i < 3; ++i) {
-			if (e[i])
-				(void)hipGraphExecDestroy(e[i]);
-			if (g[i])
-				(void)hipGraphDestroy(g[i]);
-		}
-	}
-};
-
 // The step report in pinned memory (alpha_j, beta_{j+1}), polled for instead of waiting for the
 // stream: a stream wait and the next launch after it left the chip idle for 35 to 50 us per step.
 // Cleared to a bit pattern no computation gives; the kernel stores both values whole.
@@ -152,6 +136,8 @@ void wait_report(double* report, hipStream_t s)
 	}
 }
 
+// One Lanczos decomposition from init (any norm) with the plan's current precision. Leaves the
+// kept vectors in ws.basis(0..m).
 // noise: relative matvec noise of a reduced-precision run that an FP64 restart follows (0 for
 // a plain run); see noise_reached below.
 Decomp decompose(Plan& plan, LanczosWorkspace& ws, const double* init, int max_steps, int min_steps,
@@ -248,7 +234,7 @@ Decomp decompose(Plan& plan, LanczosWorkspace& ws, const double* init, int max_s
 		DMK_HIP_CHECK(hipMemsetAsync(ws.jdev(), 0, sizeof(int), s)); // before the first captured step
 		// The captured steps report into host[2], host[3]; host[0], host[1] are the first step's.
 		double*    report = host + 2;
-		StepGraphs sg;
+		StepGraphs sg(s);
 		for (int p = 0; p < 3; ++p) {
 			double* v0 = ws.ring((p + 2) % 3);
 			double* v1 = ws.ring(p);

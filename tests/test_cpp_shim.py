@@ -34,6 +34,16 @@ def test_pool_cache_on_cpu():
     assert "all checks passed" in r.stdout
 
 
+def test_lanczos_step_on_cpu():
+    """The host side of the captured Lanczos steps (lanczos_step.h) on stand-ins for the HIP calls:
+    no graph is destroyed while the stream still runs its last launch, on any way out."""
+    _build()
+    exe = os.path.join(CPP, "_build", "test_lanczos_step")
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, r.stdout + r.stderr
+    assert "all checks passed" in r.stdout
+
+
 def test_pool_counters_export_without_gpu():
     """dmk_pool_counters is host-only bookkeeping: callable without a GPU, no stale releases."""
     import dmrgpp_amd as dm
