@@ -44,7 +44,7 @@ void launch_lanczos_update_step(double* v2, const double* v1, const double* v0, 
                                 const double* B, const int* jdev, int64_t n, const double* pdot,
                                 double* pnorm, hipStream_t s);
 void launch_finish_step(double* v2, double* basis, int64_t n, const double* pnorm, const double* A,
-                        double* B, const int* jdev, int maxn, double* host, hipStream_t s);
+                        double* B, const int* jdev, int maxn, uint64_t* report, hipStream_t s);
 void launch_copy(double* y, const double* x, int64_t n, hipStream_t s);
 
 LanczosWorkspace::~LanczosWorkspace()
@@ -97,29 +97,13 @@ struct Decomp {
 	double              energy  = 0;
 };
 
-// The step report in pinned memory (alpha_j, beta_{j+1}), polled for instead of waiting for the
-// stream: a stream wait and the next launch after it left the chip idle for 35 to 50 us per step.
-// Cleared to a bit pattern no computation gives; the kernel stores both values whole.
-constexpr uint64_t kNoReport = ~uint64_t(0);
-
-void clear_report(double* report)
-{
-	for (int i = 0; i < 2; ++i)
-		__atomic_store_n(reinterpret_cast<uint64_t*>(report) + i, kNoReport, __ATOMIC_RELEASE);
-}
-
 // Returns once both values are there. Ends also when the stream has finished (then they are, or
 // its work failed) or reports an error, looked up every 50 us.
-void wait_report(double* report, hipStream_t s)
+void wait_report(const uint64_t* report, hipStream_t s)
 {
-	auto there = [&] {
-		const uint64_t* r = reinterpret_cast<const uint64_t*>(report);
-		return __atomic_load_n(r, __ATOMIC_ACQUIRE) != kNoReport
-		       && __atomic_load_n(r + 1, __ATOMIC_ACQUIRE) != kNoReport;
-	};
 	using clock = std::chrono::steady_clock;
 	auto look   = clock::now() + std::chrono::microseconds(50);
-	while (!there()) {
+	while (!report_there(report)) {
 		if (clock::now() < look)
 			continue;
 		const hipError_t e = hipStreamQuery(s);
@@ -129,9 +113,9 @@ void wait_report(double* report, hipStream_t s)
 			DMK_HIP_CHECK(e);
 		look = clock::now() + std::chrono::microseconds(50);
 	}
-	if (!there()) {
+	if (!report_there(report)) {
 		DMK_HIP_CHECK(hipStreamSynchronize(s));
-		if (!there())
+		if (!report_there(report))
 			throw std::runtime_error("lanczos: a step ended without its report");
 	}
 }
@@ -233,7 +217,7 @@ Decomp decompose(Plan& plan, LanczosWorkspace& ws, const double* init, int max_s
 		launch_copy(ws.ring(1), ws.basis(1), n, s);
 		DMK_HIP_CHECK(hipMemsetAsync(ws.jdev(), 0, sizeof(int), s)); // before the first captured step
 		// The captured steps report into host[2], host[3]; host[0], host[1] are the first step's.
-		double*    report = host + 2;
+		uint64_t*  report = reinterpret_cast<uint64_t*>(host + 2);
 		StepGraphs sg(s);
 		for (int p = 0; p < 3; ++p) {
 			double* v0 = ws.ring((p + 2) % 3);
@@ -271,9 +255,9 @@ Decomp decompose(Plan& plan, LanczosWorkspace& ws, const double* init, int max_s
 			DMK_HIP_CHECK(hipGraphLaunch(sg.e[j % 3], s));
 			wait_report(report, s);
 			d.matvecs++;
-			d.a[size_t(j)] = report[0];
+			d.a[size_t(j)] = report_value(report[0]);
 			if (j + 1 < maxn)
-				d.b[size_t(j + 1)] = report[1];
+				d.b[size_t(j + 1)] = report_value(report[1]);
 			const double e     = tridiag_eigenvalue(d.a.data(), d.b.data(), j + 1, 0);
 			const double delta = std::fabs(e - eold);
 			eold               = e;

@@ -5,6 +5,7 @@
 // workgroup, and a single workgroup folds the partials in index order. The same n always gives
 // bitwise the same result.
 #include "dmk_internal.h"
+#include "lanczos_step.h"
 
 #include <hip/hip_runtime.h>
 
@@ -235,7 +236,7 @@ __global__ __launch_bounds__(kRedThreads) void lanczos_update_step_kernel(
 __global__ __launch_bounds__(kRedThreads) void finish_step_kernel(
     double* __restrict__ v2, double* __restrict__ basis, int64_t n, const double* __restrict__ pnorm,
     const double* __restrict__ A, double* __restrict__ B, const int* __restrict__ jdev, int maxn,
-    double* __restrict__ host)
+    uint64_t* __restrict__ report)
 {
 	const int     j      = *jdev;
 	const double  beta   = sqrt(partials_sum(pnorm, kRedBlocks));
@@ -250,9 +251,9 @@ __global__ __launch_bounds__(kRedThreads) void finish_step_kernel(
 	if (threadIdx.x == 0 && blockIdx.x == 0) {
 		if (j + 1 < maxn)
 			B[j + 1] = beta;
-		// Seen by the host while the kernel still runs (it polls; see lanczos.cpp).
-		__hip_atomic_store(host, A[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-		__hip_atomic_store(host + 1, beta, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+		// Seen by the host while the kernel still runs (it polls; see lanczos_step.h).
+		__hip_atomic_store(report, report_word(A[j]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+		__hip_atomic_store(report + 1, report_word(beta), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 	}
 }
 
@@ -335,11 +336,11 @@ void launch_lanczos_update_step(double* v2, const double* v1, const double* v0, 
 }
 
 void launch_finish_step(double* v2, double* basis, int64_t n, const double* pnorm, const double* A,
-                        double* B, const int* jdev, int maxn, double* host, hipStream_t s)
+                        double* B, const int* jdev, int maxn, uint64_t* report, hipStream_t s)
 {
 	const unsigned grid = std::min(grid_for(n), unsigned(kRedBlocks));
 	hipLaunchKernelGGL(finish_step_kernel, dim3(grid), dim3(kRedThreads), 0, s, v2, basis, n, pnorm,
-	                   A, B, jdev, maxn, host);
+	                   A, B, jdev, maxn, report);
 }
 
 void launch_copy(double* y, const double* x, int64_t n, hipStream_t s)

@@ -2,6 +2,7 @@
 // HIP calls it makes: a stream whose last graph launch is still running until somebody waits.
 #include "lanczos_step.h"
 
+#include <cstdint>
 #include <cstdio>
 #include <cstdlib>
 
@@ -60,6 +61,25 @@ int main()
 		}
 		check(g_destroyed == 2 * captured, "every graph is destroyed once");
 		check(!g_running, "the stream's work is done when the owner is gone");
+	}
+	// Every value is a report, whatever its bits, and comes back: numbers as they were, any NaN as
+	// a NaN.
+	const uint64_t words[] = { 0, 1, 0x3ff0000000000000, 0xbff8000000000001, 0x7fefffffffffffff,
+		                   0x7ff0000000000000, 0xfff0000000000000, 0x7ff8000000000000,
+		                   0xfff8000000000000, 0x7fffffffffffffff, 0xfffffffffffffffe, ~uint64_t(0) };
+	for (const uint64_t w : words) {
+		const double v = dmk::report_value(w);
+		uint64_t     r[2];
+		for (int first = 0; first < 2; ++first) {
+			dmk::clear_report(r);
+			check(!dmk::report_there(r), "a cleared report is not there");
+			r[first] = dmk::report_word(v);
+			check(!dmk::report_there(r), "half a report is not there");
+			r[1 - first] = dmk::report_word(1.5);
+			check(dmk::report_there(r), "a report of any two values is there");
+			const double back = dmk::report_value(r[first]);
+			check(v != v ? back != back : dmk::report_word(back) == w, "a value comes back");
+		}
 	}
 	if (g_failed)
 		return EXIT_FAILURE;

@@ -159,3 +159,16 @@ def test_gpu_lanczos_graph_replays_match_eager(precision):
     # Two graph solves in a row (fresh captures) give the same result again.
     rg2, zg2 = gpu_lanczos(prob, init, precision=precision, graph=1)
     assert rg2["energy"] == rg["energy"] and np.array_equal(zg2, zg)
+
+
+@pytest.mark.gpu
+def test_gpu_lanczos_start_vector_of_0xff():
+    # Memory filled with 0xff is a vector of NaNs whose payload survives arithmetic: the captured
+    # steps return what the eager ones do, and end.
+    prob = _qn(2, {-2: 30, 0: 50, 2: 30})
+    init = np.frombuffer(b"\xff" * (8 * prob.n), dtype=np.float64)
+    eager, z0 = gpu_lanczos(prob, init, max_steps=6, graph=0)
+    graph, z1 = gpu_lanczos(prob, init, max_steps=6, graph=1)
+    assert np.isnan(z0).all() and np.isnan(z1).all()
+    assert graph["steps"] == eager["steps"]
+    np.testing.assert_equal(graph["energy"], eager["energy"])
