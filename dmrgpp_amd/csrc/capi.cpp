@@ -410,10 +410,7 @@ int dmk_get_tuning(const dmk_handle* handle, dmk_tuning* tuning)
 	return guarded([&] {
 		if (!handle || !handle->plan || !tuning)
 			throw std::invalid_argument("dmk_get_tuning: null argument");
-		// Shapes that the rule picked are not reported: the caller gets the mode's base, in which
-		// any one value can be changed for dmk_set_tuning.
-		const dmk::Tuning& t = handle->plan->tuning();
-		to_c(t.by_rule ? dmk::default_tuning(handle->plan->precision()) : t, tuning);
+		to_c(handle->plan->tuning(), tuning);
 		return DMK_OK;
 	});
 }
@@ -434,7 +431,7 @@ int dmk_set_tuning(dmk_handle* handle, const dmk_tuning* tuning)
 		t.depth  = tuning->prefetch == 0 ? 1 : tuning->prefetch;
 		t.kchunk = tuning->kchunk == 0 ? 1 : tuning->kchunk;
 		t.persist = tuning->persist;
-		plan_of(handle).retune(t);
+		plan_of(handle).set_tuning(t);
 		return DMK_OK;
 	});
 }

@@ -1114,7 +1114,7 @@ std::string Plan::histogram_key() const
 	return key;
 }
 
-void Plan::retune(const Tuning& t)
+void Plan::check_tuning(const Tuning& t) const
 {
 	// 64 / 128 in every mode; FP64 and FP32 also take 96 x 96, 96 x 64 and 64 x 96, and the
 	// 32-wide tiles 32 x {32, 64, 128} and {64, 128} x 32.
@@ -1146,6 +1146,36 @@ void Plan::retune(const Tuning& t)
 	        || t.bm1 == 96 || t.bn1 == 96 || t.bm2 == 96 || t.bn2 == 96))
 		throw std::invalid_argument("dmk tuning: kchunk 2 takes FP64 / FP32 tiles of 32 or 64 "
 		                            "rows each way");
+}
+
+void Plan::set_tuning(const Tuning& t)
+{
+	if (tuning_.by_rule) {
+		// The caller had the rule's shapes reported and may have changed a part of them only. Where the
+		// rest does not go with it, that rest is the base's, with which every tile shape, load
+		// depth and K chunk that the mode has goes.
+		try {
+			check_tuning(t);
+		} catch (const std::invalid_argument&) {
+			const Tuning base = default_tuning(precision_);
+			Tuning       u    = t;
+			auto         give = [&](int Tuning::* f) {
+                                if (u.*f == tuning_.*f)
+                                        u.*f = base.*f;
+			};
+			for (auto f : { &Tuning::bm1, &Tuning::bn1, &Tuning::bm2, &Tuning::bn2, &Tuning::splitk,
+			                &Tuning::xcd, &Tuning::mfma32, &Tuning::depth, &Tuning::kchunk })
+				give(f);
+			retune(u);
+			return;
+		}
+	}
+	retune(t);
+}
+
+void Plan::retune(const Tuning& t)
+{
+	check_tuning(t);
 	if (stream_)
 		DMK_HIP_CHECK(hipStreamSynchronize(stream_));
 	tuning_                 = t;

@@ -86,8 +86,7 @@ struct StageTables {
 	void               release();
 };
 
-// The base tuning of a precision mode: where the autotuner starts, and what a handle whose
-// launch shapes nobody chose reports.
+// The base tuning of a precision mode: where the autotuner starts.
 Tuning default_tuning(int precision);
 
 // Whether the present blocks (both factors non-null) live in device or managed memory: true when
@@ -133,6 +132,10 @@ public:
 	// belongs to the current precision mode: set_precision switches to the tuning last set
 	// (or autotuned, or cached, or default) for the mode it selects.
 	void          retune(const Tuning& t);
+	// retune with a tuning that a caller chose, possibly by changing a part of the reported one.
+	void          set_tuning(const Tuning& t);
+	// Throws std::invalid_argument for what the current mode does not take.
+	void          check_tuning(const Tuning& t) const;
 	const Tuning& tuning() const { return tuning_; }
 
 	// Times candidate tunings on this problem (iters matvecs each, current precision) and keeps

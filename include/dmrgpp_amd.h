@@ -199,8 +199,9 @@ int dmk_get_info(const dmk_handle* handle, dmk_info* info);
  * BatchedGemmKokkos.h:110-130). dmk_set_tuning rebuilds the launch tables. A tuning belongs to
  * the handle's current precision mode: dmk_set_precision switches to the tuning last set or
  * autotuned for the selected mode (else the cached one, else shapes that a rule picks for the
- * problem's block sizes). While the rule's shapes are in use, dmk_get_tuning gives the mode's
- * base tuning, a valid starting point for dmk_set_tuning; dmk_info counts what runs. */
+ * problem's block sizes). dmk_get_tuning gives the tuning that runs (several vectors in one launch
+ * may run larger tiles of the rule's, with the same results). Any part of it can be changed for
+ * dmk_set_tuning: values of the rule's that do not go with the change give way to the mode's base. */
 int dmk_get_tuning(const dmk_handle* handle, dmk_tuning* tuning);
 int dmk_set_tuning(dmk_handle* handle, const dmk_tuning* tuning);
 

@@ -358,11 +358,49 @@ def test_gpu_rule_shapes(size):
         op.sync()
         assert np.array_equal(dY.download(n), one), prec
         if prec == "fp64" and size <= 1700:
-            op.set_tuning(**op.tuning())
+            op.set_tuning(stage1_tile_m=64, stage1_tile_n=64, stage2_tile_m=64, stage2_tile_n=64,
+                          splitk=2048, xcd_order=1, mfma32=0, prefetch=1, kchunk=1, persist=0)
             op.apply_Htarget(dX, dy)
             op.sync()
             assert np.array_equal(dy.download(), one)
         op.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("size", [97, 1900, 2400])
+def test_gpu_tuning_reports_what_runs(size):
+    # On a handle with the rule's shapes the reported tuning, set back, changes nothing; and a part
+    # of it can be changed to any value that the mode takes (at 1900 FP64 has two-chunk stages, which
+    # 128-wide tiles do not take; at 2400 FP32 has 96-wide tiles, which two-chunk stages do not).
+    rng = np.random.default_rng(size)
+    blocks = {(0, 0, k): (np.asfortranarray(rng.uniform(-1, 1, (size, size))),
+                          np.asfortranarray(np.eye(size))) for k in range(2)}
+    prob = dm.KronProblem(L=[size], R=[size], nC=2, blocks=blocks)
+    x = rng.uniform(-1, 1, prob.n)
+    dx, dy = dm.DeviceArray.from_host(x), dm.DeviceArray(prob.n)
+    for prec, tol in (("fp64", 1e-12), ("fp32", 1e-5), ("bf16x3", 1e-4)):
+        def run(op):
+            op.apply_Htarget(dx, dy)
+            op.sync()
+            return dy.download()
+        op = dm.BatchedGemm(prob, prec)
+        ruled, shapes, one = op.tuning(), op.info(), run(op)
+        op.set_tuning(**ruled)
+        assert op.tuning() == ruled
+        for key in ("split_tasks", "ws_elems"):
+            assert op.info()[key] == shapes[key]
+        assert np.array_equal(run(op), one), prec
+        op.close()
+        changes = [dict(stage1_tile_m=128, stage1_tile_n=128), dict(prefetch=2), dict(mfma32=1)]
+        if prec != "bf16x3":
+            changes += [dict(kchunk=2), dict(stage2_tile_m=96, stage2_tile_n=96)]
+        for change in changes:
+            op = dm.BatchedGemm(prob, prec)
+            op.set_tuning(**change)
+            got = op.tuning()
+            assert {k: got[k] for k in change} == change
+            assert rel_err(run(op), one) < tol, (prec, change)
+            op.close()
 
 
 @pytest.mark.gpu
