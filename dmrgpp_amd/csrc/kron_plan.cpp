@@ -871,13 +871,22 @@ Tuning Plan::rule_tuning(int precision) const
 		t.kchunk = kchunk;
 	};
 	if (precision == PREC_BF16X3) {
-		// Two waves per SIMD at most: the largest tiles, once they fill the chip, read the least LDS
-		// per MFMA (Hubbard 3072: 128 x 128 tiles 1107 us, 128 x 64 1190).
-		t.mfma32 = t2 < 2.5 ? 1 : 0;
-		t.splitk = t2 < 2.5 || t2 >= 5 ? 2048 : 0;
-		if (t2 < 2.5)
+		// Pieces of 1024 elements of k as in the base tuning, and its MFMA form: the FP32 accumulator
+		// of a piece then rounds as often as with the base shapes, and the results are the same
+		// bit for bit. Longer pieces are up to 12 % faster (spin 1024: 2048 elements 82 us, 1024
+		// 92; spin 2048: no split 308, 1024 314; Hub. 3072: 2048 elements 1068, 1024 1138) and
+		// err more (spin 2048: 5.06e-6 against 64 bits, 5.02e-6; spin 1024 5.18e-6, 5.17e-6).
+		// A second set of accumulators, added to every 512 k, takes the registers of a wave per
+		// SIMD at 128 x 64 (spin 2048 318 -> 333 us) and a third of the speed at 128 x 128.
+		t.splitk = 1024;
+		// us at 64 x 64 / 128 x 64 / 128 x 128: Hub. 400 (t2 0.4) 38 / 46 / 65, spin 1024 (0.8) 92 / 96 /
+		// 111, spin 1400 (1.5) 156 / 139 / 140, Hub. 1400 (1.8) 138 / 137 / 141, spin 1700 (2.1)
+		// 218 / 201 / 211, Hub. 1700 (2.7) 223 / 222 / 222, spin 2048 (3.1) 368 / 329 / 314,
+		// Hub. 2048 (3.6) 330 / 315 / 300, spin 2700 (4.9) 726 / 624 / 559, Hub. 3072 (7.0) 1476 /
+		// 1285 / 1138: the largest tiles, once they fill the chip, read the least LDS per MFMA.
+		if (t2 < 1.5)
 			shape(64, 64, 64, 64, 2, 1);
-		else if (t2 < 5)
+		else if (t2 < 3)
 			shape(128, 64, 128, 64, 1, 1);
 		else
 			shape(128, 128, 128, 128, 1, 1);
@@ -965,8 +974,13 @@ Plan::TileSet Plan::tile_set(int nvec)
                 w.bn2 = std::max(w.bn2, bn);
 	};
 	if (precision_ == PREC_BF16X3) {
-		if (t2 >= 2.5)
+		// The single vector's classes; the sums are the same at either depth.
+		if (t2 >= 3)
+			tiles(128, 128);
+		else if (t2 >= 1.5)
 			tiles(128, 64);
+		if (t2 >= 1.5)
+			w.depth = 1;
 	} else {
 		if (t2 >= 8)
 			tiles(64, 64);
