@@ -892,22 +892,28 @@ Tuning Plan::rule_tuning(int precision) const
 			shape(128, 128, 128, 128, 1, 1);
 		return t;
 	}
-	// FP64 below t2 = 3 keeps the base tuning's order of summation (single K chunks, split-k 2048),
-	// so its results are the base tuning's bit for bit, whatever the tiles; a Davidson run that
-	// starts far from its state amplifies any difference. Up to 4 % slower there than free choice.
+	// FP64 keeps the base tuning's pieces (split-k 2048) everywhere: with 4096 the matvec is at most 2 %
+	// faster (spin 2048 1067 / 1069 us, spin 1900 840 / 853, spin 2700 2096 / 2100) and errs a third
+	// more (2.60e-15 against 64 bits, 1.95e-15). Two-chunk stages add the products of a piece in
+	// another order. They win 4 to 7 % at 2.6 to 4 tiles per CU (us with 64 x 32 tiles and two-chunk
+	// stages / the best with single chunks: spin 1900 (t2 2.6) 853 / 875, spin 2048 (3.1) 1069 /
+	// 1129, Hub. 2048 (3.6) 855 / 877, spin 2400 (4.0) 958 / 972), at most 2 % below, and lose from
+	// 4.2 on (Hub. 2200 (4.3) 1818 / 1782, spin 2700 (4.9) 2100 / 2062, Hub. 3072 (7.0) 4300 / 4169).
+	// They are taken from t2 = 3: below, and from 4.2 on, results are the base tuning's bit for
+	// bit, whatever the tiles, at a cost of up to 3 % between 2.5 and 3.
 	const bool f64 = precision == PREC_FP64;
 	if (f64) {
-		t.splitk = t2 < 3 ? 2048 : 4096;
+		t.splitk = 2048;
 		if (t1 < 10 && t2 < 1.9)
 			shape(32, 32, 32, 32, 2, 1);
 		else if (t2 < 2.5)
 			shape(32, 64, 32, 32, 2, 1);
 		else if (t2 < 3)
 			shape(64, 32, 64, 32, 2, 1);
-		else if (t2 < 5)
+		else if (t2 < 4.2)
 			shape(64, 32, 64, 32, 1, 2);
 		else
-			shape(64, 64, 64, 64, 1, 2);
+			shape(64, 64, 64, 64, 1, 1);
 		return t;
 	}
 	if (t1 < 10 && t2 < 1.9) {

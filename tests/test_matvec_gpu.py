@@ -334,8 +334,8 @@ def test_gpu_balanced_launch_multi_vector(prec):
 def test_gpu_rule_shapes(size):
     # One patch of size x (size + 3) per class of the launch-shape rule (0.02 to 5.6 tiles of
     # 64 x 64 per CU): every precision against numpy with the modes' usual bounds, several vectors
-    # in one launch bitwise the single vector's, and FP64 below three tiles per CU and BF16x3
-    # bitwise the base tuning's.
+    # in one launch bitwise the single vector's, and FP64 outside 3 to 4.2 tiles per CU and
+    # BF16x3 bitwise the base tuning's.
     rng = np.random.default_rng(size)
     L, R = size, size + 3
 
@@ -357,7 +357,7 @@ def test_gpu_rule_shapes(size):
         op.apply_multi(dX, dY, nvec)
         op.sync()
         assert np.array_equal(dY.download(n), one), prec
-        if prec == "fp64" and size <= 1700:
+        if prec == "fp64" and size in (97, 700, 1410, 1700, 2400):
             op.set_tuning(stage1_tile_m=64, stage1_tile_n=64, stage2_tile_m=64, stage2_tile_n=64,
                           splitk=2048, xcd_order=1, mfma32=0, prefetch=1, kchunk=1, persist=0)
             op.apply_Htarget(dX, dy)
@@ -373,14 +373,16 @@ def test_gpu_rule_shapes(size):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("prec,cols", [("bf16x3", 16), ("bf16x3", 1000), ("bf16x3", 2240)])
-def test_gpu_long_sums_are_cut(prec, cols):
+@pytest.mark.parametrize("prec", ["fp64", "fp32", "bf16x3"])
+@pytest.mark.parametrize("cols", [16, 1000, 2240])
+def test_gpu_long_sums_are_cut(cols, prec):
     # A contraction of 6 x 1400 elements whose first product is 1 and whose others are so small that
-    # one MFMA's worth of them (32 products of bf16) is below half a unit of the accumulator: a piece
+    # one MFMA's worth of them (4 products, 32 of bf16) is below half a unit of the accumulator: a piece
     # that starts with the 1 loses the rest of itself, and no other piece loses anything. So the
     # error tells how long the pieces are: at most the base tuning's.
     K, terms = 1400, 6
-    piece, eps, unit = {"bf16x3": (1024, 2.0 ** -30, 2.0 ** -24)}[prec]
+    piece, eps, unit = {"fp64": (2048, 2.0 ** -56, 2.0 ** -53), "fp32": (2048, 2.0 ** -27, 2.0 ** -24),
+                        "bf16x3": (1024, 2.0 ** -30, 2.0 ** -24)}[prec]
     first = np.full((K, K), eps, order="F")
     first[:, 0] = 1.0
     rest = np.full((K, K), eps, order="F")
@@ -396,8 +398,8 @@ def test_gpu_long_sums_are_cut(prec, cols):
     # Rows are padded to 64, and the range is cut into equal pieces of at least `piece` elements.
     total = terms * 1408
     longest = total / (total // piece) + 64
-    want = 1.0 + (terms * K - 1) * eps
-    assert np.abs(got - want).max() <= longest * eps + (total // piece) * unit
+    tail = (terms * K - 1) * eps
+    assert np.abs((got - 1.0) - tail).max() <= longest * eps + (total // piece) * unit
 
 
 @pytest.mark.gpu
