@@ -952,9 +952,18 @@ void Plan::release_multi_sets()
 }
 
 // With several vectors per launch the chip is filled sooner, and the larger tiles pay at smaller
-// problems. FP64, eight vectors, us per launch with the single vector's tiles / this rule's / the
-// best of all: Hubbard m = 400 (t2 0.4) 134 / 135 / 133, Heisenberg 1024 (0.8) 1392 / 1298 / 1242,
-// Hubbard 1400 (2.0) 2972 / 2537 / 2491, Hubbard 2048 (3.6) 7462 / 7138 / 7064.
+// problems, unless the blocks are so small that those are mostly padding. us per launch with the
+// single vector's tiles / this rule's / the base tuning's:
+//   FP64     Hub. 400 (t2 0.4) x 8 131 / 130 / 207, spin 1024 (0.8) x 4 679 / 677 / 688, x 8 1404 /
+//            1265 / 1270, Hub. 1024 (1.7) x 3 633 / 628 / 668, x 8 1721 / 1588 / 1586, Hub. 1400
+//            (1.8) x 2 673 / 675 / 637, x 3 1017 / 990 / 983, x 4 1364 / 1255 / 1266, x 8 2766 /
+//            2415 / 2422, spin 1400 (1.5) x 8 3298 / 2941 / 2980, Hub. 2048 (3.6) x 8 7383 / 7049 / 7087
+//   BF16x3   spin 1024 x 8 440 / 384 / 443, Hub. 1024 x 4 311 / 261 / 310, Hub. 1400 x 8 907 / 779 /
+//            908, Hub. 2048 x 8 1915 / 1922 / 2186
+// Padding: 128 x 128 tiles cover 1.2 to 1.5 times the area of 64 x 64 ones there, and 2.8 times on
+// Hub. 400, whose patches are 1 to 80 wide (BF16x3 x 12: 103 us with the single vector's tiles, 144
+// with 128 x 128; x 8, 128 x 64, 1.6 times: 79 and 94; FP64 x 16, 64 x 64 against 32 x 32, 1.8
+// times: 232 and 250).
 Plan::TileSet Plan::tile_set(int nvec)
 {
 	TileSet s;
@@ -988,21 +997,34 @@ Plan::TileSet Plan::tile_set(int nvec)
 		if (t2 >= 1.5)
 			w.depth = 1;
 	} else {
-		if (t2 >= 8)
+		const bool f64 = precision_ == PREC_FP64;
+		if (t2 >= (f64 ? 6 : 8))
 			tiles(64, 64);
 		else if (t2 >= 4)
 			tiles(64, 32);
-		// FP64 sums in the same order at either depth; FP32 folds its sums at one depth only.
-		if (precision_ == PREC_FP64 && t2 >= 4)
-			w.depth = tuning_.kchunk == 1 ? 2 : 1;
+		// FP64 sums in the same order at either depth, and 64 x 64 tiles run faster with two LDS
+		// stages; FP32 folds its sums at one depth only, so it keeps the single vector's.
+		if (f64 && t2 >= 6)
+			w.depth = 1;
 	}
 	if (w.bm1 == s.bm1 && w.bn1 == s.bn1 && w.bm2 == s.bm2 && w.bn2 == s.bn2) {
 		s.depth = w.depth;
 		return s;
 	}
+	auto covered = [&](int bm, int bn) { // by stage 2's tiles
+		double a = 0;
+		for (const PTask& t : t2_tasks_)
+			a += double((t.m + bm - 1) / bm * bm) * double((t.n + bn - 1) / bn * bn);
+		return a;
+	};
+	if (covered(w.bm2, w.bn2) > 1.55 * covered(s.bm2, s.bn2))
+		return s;
 	for (const TileSet& m : multi_sets_)
-		if (m.bm1 == w.bm1 && m.bn1 == w.bn1 && m.bm2 == w.bm2 && m.bn2 == w.bn2)
-			return m;
+		if (m.bm1 == w.bm1 && m.bn1 == w.bn1 && m.bm2 == w.bm2 && m.bn2 == w.bn2) {
+			s       = m;
+			s.depth = w.depth;
+			return s;
+		}
 	// The lists are uploaded on first use, which a stream capture cannot record: there the single
 	// vector's tiles serve.
 	hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;

@@ -373,6 +373,37 @@ def test_gpu_rule_shapes(size):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("nvec", [2, 3, 5, 9, 24])
+@pytest.mark.parametrize("small", [False, True])
+def test_gpu_rule_shapes_of_several_vectors(small, nvec):
+    # The tiles of a launch for several vectors (0.9 to 11 tiles of 64 x 64 per CU of one 700 x 690
+    # patch; patches of at most 40 x 40, where larger tiles would be padding): every vector bitwise
+    # as alone, in every precision and again with other numbers of vectors in between.
+    sizes = list(range(1, 41)) if small else [700]
+    rng = np.random.default_rng(nvec)
+    blocks = {(i, i, k): (np.asfortranarray(rng.uniform(-1, 1, (m, m))),
+                          np.asfortranarray(rng.uniform(-1, 1, (m - m // 70,) * 2)))
+              for i, m in enumerate(sizes) for k in range(3)}
+    prob = dm.KronProblem(L=sizes, R=[m - m // 70 for m in sizes], nC=3, blocks=blocks)
+    n = prob.n
+    X = rng.uniform(-1, 1, (nvec, n))
+    dX, dx = dm.DeviceArray.from_host(X.ravel()), dm.DeviceArray(n)
+    dY, dy = dm.DeviceArray(nvec * n), dm.DeviceArray(n)
+    for prec in ("fp64", "fp32", "bf16x3"):
+        op = dm.BatchedGemm(prob, prec)
+        for count in (nvec, nvec // 2 + 1, nvec):
+            op.apply_multi(dX, dY, count)
+            op.sync()
+            got = dY.download(count * n).reshape(count, n)
+            for v in (0, count // 2, count - 1):
+                dx.upload(X[v])
+                op.apply_Htarget(dx, dy)
+                op.sync()
+                assert np.array_equal(got[v], dy.download()), (prec, count, v)
+        op.close()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("prec", ["fp64", "fp32", "bf16x3"])
 @pytest.mark.parametrize("cols", [16, 1000, 2240])
 def test_gpu_long_sums_are_cut(cols, prec):
