@@ -155,9 +155,11 @@ void gemm_vbatch(bool cplx, char transa, char transb, const int* m, const int* n
 	}
 	if (ents.empty())
 		return;
+	const bool alpha_zero = alpha[0] == 0.0 && (!cplx || alpha[1] == 0.0); // A and B are not read
 	for (const VbEntry& e : ents)
-		if (!panel_ld_fits(panel_ld(e.k)))
-			throw std::runtime_error("gemm_vbatch: a contraction is too long for the panel kernel");
+		if (!alpha_zero && e.k > kVbMaxK)
+			throw std::runtime_error("gemm_vbatch: a contraction is longer than "
+			                         + std::to_string(kVbMaxK));
 	VbLaunch p {};
 	p.cplx      = cplx;
 	p.ta        = ta;
@@ -181,7 +183,7 @@ void gemm_vbatch(bool cplx, char transa, char transb, const int* m, const int* n
 		throw std::runtime_error("gemm_vbatch: batch too large for one launch");
 	const RunLists lists   = list_runs(ents, p.tile);
 	const size_t   scalar  = (cplx ? 2 : 1) * sizeof(double);
-	const bool     through = outputs_meet_inputs(ents, ta, tb, scalar);
+	const bool     through = !alpha_zero && outputs_meet_inputs(ents, ta, tb, scalar);
 
 	const size_t ebytes = ents.size() * sizeof(VbEntry), rbytes = lists.runs.size() * sizeof(VbRun);
 	void*        host = nullptr;

@@ -42,6 +42,9 @@ struct VbLaunch {
 // Largest leading dimension whose byte offsets within a tile fit 32 bits (64 rows, 16 bytes).
 constexpr int kVbNarrowLd = 1 << 21;
 
+// Longest contraction that the entry points take.
+constexpr int kVbMaxK = 1 << 21;
+
 // runs: eight lists of nruns each, by position (filled up with first = INT32_MAX); `longest`
 // positions in the longest list.
 void launch_vb_gemm(const VbLaunch& p, const VbEntry* entries, const VbRun* runs, int nruns,
@@ -51,7 +54,8 @@ void launch_vb_copy_back(const VbEntry* entries, int nentries, bool cplx, hipStr
 
 // C_e = alpha op(A_e) op(B_e) + beta C_e for every entry e of every group (m, n, k, lda, ldb,
 // ldc per group; pointers per entry, device memory, expanded in group order). cplx selects
-// interleaved complex scalars (alpha, beta then point to (re, im) pairs). Synchronous.
+// interleaved complex scalars (alpha, beta then point to (re, im) pairs). Synchronous. k is at most
+// kVbMaxK unless alpha is 0.
 void gemm_vbatch(bool cplx, char transa, char transb, const int* m, const int* n, const int* k,
                  const double* alpha, const double* const* a, const int* lda,
                  const double* const* b, const int* ldb, const double* beta, double* const* c,

@@ -373,8 +373,8 @@ int dmk_density_svd_d(int nblocks, const int64_t* rows, const int64_t* cols,
  * call. For every entry e of every group g: C_e = alpha op(A_e) op(B_e) + beta C_e, column major,
  * op from transa/transb ('N', 'T', or 'C' = conjugate transpose as in BLAS). m/n/k/lda/ldb/ldc
  * and group_size have group_count entries; a/b/c hold one device pointer per entry, in group
- * order (host arrays). C is not read when beta == 0. Runs on the MFMA grouped kernel (FP64);
- * synchronous. Used by the sweep driver for the wave-function transformation GEMMs
+ * order (host arrays). C is not read when beta == 0, A and B are not when alpha == 0; otherwise k
+ * is at most 2^21. Runs on FP64 MFMAs, from the caller's matrices into the caller's C; synchronous. Used by the sweep driver for the wave-function transformation GEMMs
  * (WftAccelBlocks.h:162-322). */
 int dmk_gemm_vbatch_d(char transa, char transb, const int* m_array, const int* n_array,
                       const int* k_array, double alpha, const double* const* a_array,

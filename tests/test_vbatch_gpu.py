@@ -96,6 +96,23 @@ def test_gpu_vbatch_alpha_zero_scales_c_only():
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("cplx", [False, True])
+def test_gpu_vbatch_alpha_zero_takes_any_contraction(cplx):
+    # With alpha = 0 the operands are not read, whatever k says; a product that long is refused by
+    # the entry point's limit, and C is left alone.
+    w = 2 if cplx else 1
+    m, n, k = 3, 2, (1 << 21) + 1
+    C = np.random.default_rng(6).uniform(-1, 1, w * m * n)
+    dA, dC = dm.DeviceArray(1), dm.DeviceArray.from_host(C)
+    group = [(m, n, k, m, k, m, [(dA.ptr, dA.ptr, dC.ptr)])]
+    with pytest.raises(dm.DmkError, match="contraction is longer than 2097152"):
+        dm.gemm_vbatch("N", "N", group, alpha=1.0, beta=3.0, cplx=cplx)
+    np.testing.assert_array_equal(dC.download(), C)
+    dm.gemm_vbatch("N", "N", group, alpha=0.0, beta=3.0, cplx=cplx)
+    np.testing.assert_array_equal(dC.download(), 3.0 * C)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("cplx", [False, True])
 @pytest.mark.parametrize("transa,transb", [("N", "N"), ("N", "T"), ("T", "N"), ("T", "T")])
 def test_gpu_vbatch_large_batch_tiles(transa, transb, cplx):
     # Enough tiles for the 64 x 64 kernel (2048 of them), k at every remainder of a 16-element chunk
