@@ -11,11 +11,11 @@
 
 #include "dmk_internal.h"
 #include "pool.h"
+#include "vbatch_plan.h"
 
 #include <algorithm>
 #include <cstdint>
 #include <cstring>
-#include <numeric>
 #include <stdexcept>
 #include <string>
 #include <vector>
@@ -40,83 +40,6 @@ int trans_code(char t, const char* which)
 	default:
 		throw std::invalid_argument(std::string("gemm_vbatch: bad ") + which + " '" + t + "'");
 	}
-}
-
-constexpr int kXcds = 8;
-
-// Whether any output's memory range meets any input's (by range: interleaved submatrices count).
-bool outputs_meet_inputs(const std::vector<VbEntry>& ents, int ta, int tb, size_t scalar)
-{
-	struct Range {
-		uintptr_t lo, hi;
-		bool      out;
-	};
-	std::vector<Range> r;
-	r.reserve(3 * ents.size());
-	auto add = [&](const double* p, int rows, int cols, int ld, bool out) {
-		const uintptr_t lo = reinterpret_cast<uintptr_t>(p);
-		r.push_back(Range { lo, lo + (size_t(cols - 1) * size_t(ld) + size_t(rows)) * scalar, out });
-	};
-	for (const VbEntry& e : ents) {
-		add(e.c, e.m, e.n, e.ldc, true);
-		if (e.k > 0) {
-			add(e.a, ta ? e.k : e.m, ta ? e.m : e.k, e.lda, false);
-			add(e.b, tb ? e.n : e.k, tb ? e.k : e.n, e.ldb, false);
-		}
-	}
-	std::sort(r.begin(), r.end(), [](const Range& x, const Range& y) { return x.lo < y.lo; });
-	uintptr_t end[2] = { 0, 0 };
-	for (const Range& x : r) {
-		if (x.lo < end[x.out ? 0 : 1])
-			return true;
-		end[x.out ? 1 : 0] = std::max(end[x.out ? 1 : 0], x.hi);
-	}
-	return false;
-}
-
-// Which tiles each XCD's workgroups take (workgroup b runs on XCD b % 8): every entry's tiles, the
-// longest contractions first, in eight runs, so that neighbouring tiles share an L2; small entries
-// go whole to the XCD with the least work. The workgroups find their tiles in these lists, which
-// spares the host and the upload the tiles themselves (a few thousand per call).
-struct RunLists {
-	std::vector<VbRun> runs; // kXcds lists of nruns
-	int                nruns   = 0;
-	int64_t            longest = 0;
-};
-
-RunLists list_runs(const std::vector<VbEntry>& ents, int T)
-{
-	std::vector<int> order(ents.size());
-	std::iota(order.begin(), order.end(), 0);
-	std::stable_sort(order.begin(), order.end(),
-	                 [&](int x, int y) { return ents[size_t(x)].k > ents[size_t(y)].k; });
-	std::vector<VbRun> lists[kXcds];
-	double             load[kXcds] = {};
-	int64_t            count[kXcds] = {};
-	for (int e : order) {
-		const VbEntry& en   = ents[size_t(e)];
-		const int64_t  nt   = int64_t((en.m + T - 1) / T) * ((en.n + T - 1) / T);
-		const double   cost = double(en.k) + 32.0;
-		for (int64_t run = 0, t = 0; t < nt; ++run) {
-			const int64_t end = nt < kXcds ? nt : nt * (run + 1) / kXcds;
-			if (end == t)
-				continue;
-			const int x = int(std::min_element(load, load + kXcds) - load);
-			lists[x].push_back(VbRun { int32_t(count[x]), e, int32_t(t), int32_t(end) });
-			count[x] += end - t;
-			load[x] += cost * double(end - t);
-			t = end;
-		}
-	}
-	RunLists out;
-	for (int x = 0; x < kXcds; ++x) {
-		out.nruns   = std::max(out.nruns, int(lists[x].size()));
-		out.longest = std::max(out.longest, count[x]);
-	}
-	out.runs.assign(size_t(out.nruns) * kXcds, VbRun { INT32_MAX, 0, 0, 0 });
-	for (int x = 0; x < kXcds; ++x)
-		std::copy(lists[x].begin(), lists[x].end(), out.runs.begin() + size_t(x) * size_t(out.nruns));
-	return out;
 }
 
 } // namespace
@@ -179,11 +102,11 @@ void gemm_vbatch(bool cplx, char transa, char transb, const int* m, const int* n
 		p.wide = p.wide || e.lda > kVbNarrowLd || e.ldb > kVbNarrowLd;
 	}
 	p.tile = tiles64 < 4 * 256 ? 32 : 64;
-	if (tiles64 * double(64 / p.tile) * double(64 / p.tile) > double(0x7fffffff / kXcds))
+	if (tiles64 * double(64 / p.tile) * double(64 / p.tile) > double(0x7fffffff / kVbXcds))
 		throw std::runtime_error("gemm_vbatch: batch too large for one launch");
-	const RunLists lists   = list_runs(ents, p.tile);
+	const VbRunLists lists = vb_list_runs(ents, p.tile);
 	const size_t   scalar  = (cplx ? 2 : 1) * sizeof(double);
-	const bool     through = !alpha_zero && outputs_meet_inputs(ents, ta, tb, scalar);
+	const bool     through = !alpha_zero && vb_outputs_meet_inputs(ents, ta, tb, scalar);
 
 	const size_t ebytes = ents.size() * sizeof(VbEntry), rbytes = lists.runs.size() * sizeof(VbRun);
 	void*        host = nullptr;

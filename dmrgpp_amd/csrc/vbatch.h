@@ -42,6 +42,8 @@ struct VbLaunch {
 // Largest leading dimension whose byte offsets within a tile fit 32 bits (64 rows, 16 bytes).
 constexpr int kVbNarrowLd = 1 << 21;
 
+constexpr int kVbXcds = 8;
+
 // Longest contraction that the entry points take.
 constexpr int kVbMaxK = 1 << 21;
 

@@ -28,7 +28,6 @@ namespace dmk {
 namespace {
 
 constexpr int kVbThreads = 256;
-constexpr int kVbXcds    = 8;
 constexpr int kVbK       = 16; // chunk of k
 constexpr int kVbAhead   = 4;  // chunks in flight in registers (even: the LDS buffer of a step is static)
 
@@ -153,22 +152,22 @@ __global__ __launch_bounds__(kVbThreads) void vb_gemm_kernel(
 
 	const int     tid = threadIdx.x, lane = tid & 63;
 	// Workgroup b is position b / 8 of XCD b % 8's list; its run is the last that starts there or
-	// before (64 candidates at a time).
+	// before: 64 candidates at a time, evenly over what is left of the list, so lists of up to 4096
+	// runs take two dependent loads.
 	const int    pos  = int(blockIdx.x) / kVbXcds;
 	const VbRun* list = runs + int64_t(blockIdx.x % kVbXcds) * nruns;
-	int          run  = -1;
-	for (int r0 = 0; r0 < nruns; r0 += 64) {
-		const bool     here = r0 + lane < nruns && list[r0 + lane].first <= pos;
-		const uint64_t mask = __ballot(here);
-		run += __popcll(mask);
-		if (mask != ~uint64_t(0))
-			break;
+	int          run  = 0;
+	for (int end = nruns; end - run > 1;) {
+		const int      step  = (end - run + 63) / 64;
+		const int      at    = run + lane * step;
+		const uint64_t mask  = __ballot(at < end && list[at].first <= pos);
+		const int      below = max(__popcll(mask), 1) - 1;
+		end                  = min(end, run + (below + 1) * step);
+		run += below * step;
 	}
-	if (run < 0)
-		return;
 	const VbRun rn = list[__builtin_amdgcn_readfirstlane(run)];
 	const int   t  = rn.t0 + pos - rn.first;
-	if (t >= rn.t1)
+	if (pos < rn.first || t >= rn.t1)
 		return;
 	const VbEntry en = entries[rn.entry];
 	const int     tm = (en.m + T - 1) / T;

@@ -44,6 +44,16 @@ def test_lanczos_step_on_cpu():
     assert "all checks passed" in r.stdout
 
 
+def test_vbatch_plan_on_cpu():
+    """The batched GEMM's host planning (vbatch_plan.h): overlaps of outputs and inputs as found by
+    pairs, two or three ranges for packed operands, every tile once in the XCDs' lists."""
+    _build()
+    exe = os.path.join(CPP, "_build", "test_vbatch_plan")
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, r.stdout + r.stderr
+    assert "all checks passed" in r.stdout
+
+
 def test_pool_counters_export_without_gpu():
     """dmk_pool_counters is host-only bookkeeping: callable without a GPU, no stale releases."""
     import dmrgpp_amd as dm

@@ -142,6 +142,32 @@ def test_gpu_vbatch_large_batch_tiles(transa, transb, cplx):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("count", [1, 8, 9, 512, 513, 4097, 40000])
+def test_gpu_vbatch_many_small_entries(count):
+    # One run per entry: lists of 1 to 5000 runs per XCD (one, two and three steps of the search), sizes
+    # of one tile and, every 97th entry, several.
+    rng = np.random.default_rng(count)
+    i = np.arange(count)
+    m, n, k = 1 + i % 5, 1 + i % 3, i % 4
+    m[::97] += 60
+    A = rng.uniform(-1, 1, int((m * np.maximum(k, 1)).sum()))
+    B = rng.uniform(-1, 1, int((n * np.maximum(k, 1)).sum()))
+    dA, dB, dC = dm.DeviceArray.from_host(A), dm.DeviceArray.from_host(B), dm.DeviceArray(int((m * n).sum()))
+    dC.upload(np.full(dC.size, np.nan))
+    oa, ob, oc = (np.concatenate([[0], np.cumsum(v)]) for v in
+                  (m * np.maximum(k, 1), n * np.maximum(k, 1), m * n))
+    dm.gemm_vbatch("N", "T", [(int(m[e]), int(n[e]), int(k[e]), int(m[e]), int(n[e]), int(m[e]),
+                               [(dA.ptr + 8 * int(oa[e]), dB.ptr + 8 * int(ob[e]), dC.ptr + 8 * int(oc[e]))])
+                              for e in range(count)])
+    got = dC.download()
+    for e in range(count):
+        a = A[oa[e]:oa[e + 1]].reshape((-1, m[e]))[:k[e]]
+        b = B[ob[e]:ob[e + 1]].reshape((-1, n[e]))[:k[e]]
+        # At most three products of at most 1.
+        assert np.abs(got[oc[e]:oc[e + 1]].reshape((n[e], m[e])) - b.T @ a).max() <= 24 * 2.0 ** -53
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("wide", [False, True])
 def test_gpu_vbatch_output_over_input_and_wide_rows(wide):
     # C in the memory of A (computed through a workspace), and a leading dimension past 2^21.
