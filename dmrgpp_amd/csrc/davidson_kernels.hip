@@ -287,33 +287,39 @@ __global__ __launch_bounds__(kDT) __attribute__((amdgpu_waves_per_eu(2))) void p
 	sm.load(params, threadIdx.x);
 	const int  lane = threadIdx.x & 63;
 	const int  c = lane & 15, g = lane >> 4;
-	MlpWeights w;
-	w.load(params, c, g);
+	const bool infinite = mlp_infinite(params, lane);
 	__syncthreads();
 	const double  eps  = (sums[1] != 0.0) ? sums[0] / sums[1] : 0.0;
 	const double  unit = rms_r / sD;
 	const int64_t step = int64_t(gridDim.x) * kDT;
-	for (int64_t i0 = int64_t(blockIdx.x) * kDT + (threadIdx.x - lane); i0 < n; i0 += step) {
-		// Every lane of the wave takes part in the tiles: past the end it repeats the last element.
-		const int64_t i    = i0 + lane < n ? i0 + lane : n - 1;
-		const double  tols = olsen_elem(D[i], r[i], u[i], theta, floor_, eps);
-		float         f[kMlpIn];
-		features(D[i], r[i], u[i], theta, sD, rms_r, rms_u, tols / unit, f);
-		float y = 0.0f;
+	auto run = [&](auto w) {
+		w.load(params, c, g);
+		for (int64_t i0 = int64_t(blockIdx.x) * kDT + (threadIdx.x - lane); i0 < n; i0 += step) {
+			// Every lane of the wave takes part in the tiles: past the end it repeats the last element.
+			const int64_t i    = i0 + lane < n ? i0 + lane : n - 1;
+			const double  tols = olsen_elem(D[i], r[i], u[i], theta, floor_, eps);
+			float         f[kMlpIn];
+			features(D[i], r[i], u[i], theta, sD, rms_r, rms_u, tols / unit, f);
+			float y = 0.0f;
 #pragma unroll 1
-		for (int q = 0; q < 4; ++q) {
-			mlp_tile_fence();
-			const int   src = kMlpTile * q + c;
-			const float f0 = __shfl(f[0], src), f1 = __shfl(f[1], src);
-			const float f2 = __shfl(f[2], src), f3 = __shfl(f[3], src);
-			const float xi = g == 0 ? f0 : g == 1 ? f1 : g == 2 ? f2 : f3;
-			const float out = mlp_forward_tile(w, sm, g, xi);
-			if (g == q)
-				y = out;
+			for (int q = 0; q < 4; ++q) {
+				mlp_tile_fence();
+				const int   src = kMlpTile * q + c;
+				const float f0 = __shfl(f[0], src), f1 = __shfl(f[1], src);
+				const float f2 = __shfl(f[2], src), f3 = __shfl(f[3], src);
+				const float xi = g == 0 ? f0 : g == 1 ? f1 : g == 2 ? f2 : f3;
+				const float out = mlp_forward_tile(w, sm, g, xi);
+				if (g == q)
+					y = out;
+			}
+			if (i0 + lane < n)
+				t[i] = tols + double(y) * unit;
 		}
-		if (i0 + lane < n)
-			t[i] = tols + double(y) * unit;
-	}
+	};
+	if (infinite)
+		run(MlpWeightsInfinite {});
+	else
+		run(MlpWeights {});
 }
 
 // Features of `count` sampled elements i_q = (phase + q * stride) mod n of one iterate

@@ -49,12 +49,12 @@ struct MlpSplit {
 		m[i]          = __bf16(d);
 		l[i]          = __bf16(d - float(m[i]));
 	}
-	// For any value: past the largest bf16 the rest goes to m and l; an infinity is that value.
+	// For any finite value: past the largest bf16 the rest goes to m and l.
 	__device__ inline void set_any(int i, float v)
 	{
 		const float top = 3.3895314e38f;
 		h[i]            = __bf16(v > top ? top : v < -top ? -top : v);
-		const float d   = isinf(v) ? 0.0f : v - float(h[i]);
+		const float d   = v - float(h[i]);
 		m[i]            = __bf16(d);
 		l[i]            = __bf16(d - float(m[i]));
 	}
@@ -103,6 +103,33 @@ struct MlpWeights {
 	}
 };
 
+// The same where W2 holds an infinity, which has no parts (its products with the parts of a number
+// would be NaN where one of those is 0): layer 2 on FP32 MFMAs, its rows from global memory.
+struct MlpWeightsInfinite {
+	float        w1[kMlpBlocks];
+	const float* w2; // row c, from column 4 g on
+
+	__device__ inline void load(const float* __restrict__ params, int c, int g)
+	{
+#pragma unroll
+		for (int b = 0; b < kMlpBlocks; ++b)
+			w1[b] = params[kMlpOffW1 + (16 * b + c) * kMlpIn + g];
+		w2 = params + kMlpOffW2 + c * kMlpHidden + 4 * g;
+	}
+};
+
+// Whether W2 holds an infinity; the same in every lane of the wave. The kernels ask before they
+// load their weights and choose their loop by it: both forms in one loop do not fit three waves per
+// SIMD, and 64 loads per lane, once per wave, are in flight together.
+__device__ inline bool mlp_infinite(const float* __restrict__ params, int lane)
+{
+	bool inf = false;
+#pragma unroll 16
+	for (int i = 0; i < kMlpHidden * kMlpHidden / 64; ++i)
+		inf |= isinf(params[kMlpOffW2 + 64 * i + lane]);
+	return __ballot(inf) != 0;
+}
+
 // Biases of both layers and the output layer, in LDS.
 struct MlpSmall {
 	float b1[kMlpHidden], b2[kMlpHidden], w3[kMlpHidden];
@@ -129,15 +156,9 @@ struct MlpSmall {
 // W2's 64 they would leave three waves per SIMD, or spill).
 __device__ inline void mlp_tile_fence() { asm volatile("" ::: "memory"); }
 
-// The network's output for sample c of a tile (in every lane group); x is feature g of sample c.
-__device__ inline float mlp_forward_tile(const MlpWeights& w, const MlpSmall& sm, int g, float x)
+// h2 += W2 tanh(h1).
+__device__ inline void mlp_layer2(const MlpWeights& w, const mlp_f4 h1[kMlpBlocks], mlp_f4 h2[kMlpBlocks])
 {
-	mlp_f4 h1[kMlpBlocks], h2[kMlpBlocks];
-#pragma unroll
-	for (int b = 0; b < kMlpBlocks; ++b) {
-		h1[b] = mlp_mma(w.w1[b], x, sm.at(sm.b1, b, g));
-		h2[b] = sm.at(sm.b2, b, g);
-	}
 #pragma unroll
 	for (int s = 0; s < 2; ++s) {
 		MlpSplit v;
@@ -164,6 +185,34 @@ __device__ inline float mlp_forward_tile(const MlpWeights& w, const MlpSmall& sm
 		for (int b = 0; b < kMlpBlocks; ++b)
 			h2[b] = mlp_mma(w.w2[b][s].h, v.h, h2[b]);
 	}
+}
+
+__device__ inline void mlp_layer2(const MlpWeightsInfinite& w, const mlp_f4 h1[kMlpBlocks],
+                                  mlp_f4 h2[kMlpBlocks])
+{
+#pragma unroll
+	for (int b = 0; b < kMlpBlocks; ++b)
+#pragma unroll
+		for (int r = 0; r < 4; ++r) {
+			const float v = mlp_tanh(h1[b][r]);
+#pragma unroll
+			for (int b2 = 0; b2 < kMlpBlocks; ++b2)
+				h2[b2] = mlp_mma(w.w2[16 * b2 * kMlpHidden + 16 * b + r], v, h2[b2]);
+			mlp_tile_fence(); // a few loads at a time
+		}
+}
+
+// The network's output for sample c of a tile (in every lane group); x is feature g of sample c.
+template <typename W>
+__device__ inline float mlp_forward_tile(const W& w, const MlpSmall& sm, int g, float x)
+{
+	mlp_f4 h1[kMlpBlocks], h2[kMlpBlocks];
+#pragma unroll
+	for (int b = 0; b < kMlpBlocks; ++b) {
+		h1[b] = mlp_mma(w.w1[b], x, sm.at(sm.b1, b, g));
+		h2[b] = sm.at(sm.b2, b, g);
+	}
+	mlp_layer2(w, h1, h2);
 	float y = 0.0f;
 #pragma unroll
 	for (int b = 0; b < kMlpBlocks; ++b) {

@@ -39,27 +39,33 @@ __global__ __launch_bounds__(kT) __attribute__((amdgpu_waves_per_eu(3))) void ml
 	sm.load(params, threadIdx.x);
 	const int  lane = threadIdx.x & 63;
 	const int  c = lane & 15, g = lane >> 4;
-	MlpWeights w;
-	w.load(params, c, g);
+	const bool infinite = mlp_infinite(params, lane);
 	__syncthreads();
 	const int64_t step = int64_t(gridDim.x) * (kT / 64) * kMlpTile;
-	int64_t       s0   = (int64_t(blockIdx.x) * (kT / 64) + (threadIdx.x >> 6)) * kMlpTile;
-	auto          feature = [&](int64_t t0) {
+	const int64_t first = (int64_t(blockIdx.x) * (kT / 64) + (threadIdx.x >> 6)) * kMlpTile;
+	if (first >= count)
+		return;
+	auto feature = [&](int64_t t0) {
                 const int64_t s = t0 + c < count ? t0 + c : count - 1; // past the end: unused
                 return x[s * kMlpIn + g];
 	};
-	if (s0 >= count)
-		return;
-	float xn = feature(s0);
-	for (; s0 < count; s0 += step) {
-		mlp_tile_fence();
-		const float xi = xn;
-		if (s0 + step < count)
-			xn = feature(s0 + step);
-		const float out = mlp_forward_tile(w, sm, g, xi);
-		if (g == 0 && s0 + c < count)
-			y[s0 + c] = out;
-	}
+	auto run = [&](auto w) {
+		float xn = feature(first);
+		w.load(params, c, g);
+		for (int64_t s0 = first; s0 < count; s0 += step) {
+			mlp_tile_fence();
+			const float xi = xn;
+			if (s0 + step < count)
+				xn = feature(s0 + step);
+			const float out = mlp_forward_tile(w, sm, g, xi);
+			if (g == 0 && s0 + c < count)
+				y[s0 + c] = out;
+		}
+	};
+	if (infinite)
+		run(MlpWeightsInfinite {});
+	else
+		run(MlpWeights {});
 }
 
 // Per-workgroup partial gradient of L = (1/N) sum_s (y_s - t_s)^2 over samples

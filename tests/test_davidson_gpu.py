@@ -93,6 +93,27 @@ def test_gpu_mlp_forward_tiles(count):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("count", [1, 17, 300])
+def test_gpu_mlp_forward_infinite_and_largest_weights(count):
+    """Weights at the ends of FP32: an infinity times 0 is NaN, opposite ones cancel to NaN, one alone
+    saturates its unit, and the largest finite numbers multiply as they are."""
+    x = np.random.default_rng(count).uniform(0.5, 1.5, (count, 4)).astype(np.float32)
+    big = np.float32(np.finfo(np.float32).max)
+    # Hidden units of layer 1: 0 is exactly 0, 1 positive, 2 its negative; layer 2 unit 0 takes them.
+    for weights, want in (((np.inf, 0, 0), np.nan), ((0, np.inf, 0), 1.0), ((0, -np.inf, 0), -1.0),
+                          ((0, np.inf, np.inf), np.nan), ((np.nan, 0, 0), np.nan),
+                          ((big, 0, 0), 0.0), ((0, big, 0), 1.0)):
+        p = np.zeros(mlp_oracle.NPARAMS, dtype=np.float32)
+        p[mlp_oracle.OFF_W1:mlp_oracle.OFF_B1].reshape(64, 4)[1:3, 0] = 1.0, -1.0
+        p[mlp_oracle.OFF_W2:mlp_oracle.OFF_W2 + 3] = weights
+        p[mlp_oracle.OFF_W3] = 1.0
+        net = dm.Mlp(seed=5, capacity=1)
+        net.set_params(p)
+        np.testing.assert_array_equal(net.forward(x), np.full(count, want, dtype=np.float32))
+        net.close()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("count", [1, 15, 65, 256 * 64, 256 * 64 + 1, 3 * 256 * 64 - 5])
 def test_gpu_mlp_gradient_passes(count):
     """Remainders of a tile and a pass, and one, two and three passes per workgroup; the loss alone
