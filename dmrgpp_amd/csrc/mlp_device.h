@@ -60,25 +60,29 @@ struct MlpSplit {
 	}
 };
 
-// tanh in FP32: x + x^3 P(x^2) below 0.6 (P: minimax polynomial of (tanh(x)/x - 1)/x^2, 3e-9),
-// 1 - 2 / (1 + exp(2 x)) from the hardware exp2 and reciprocal above. Absolute error at most
-// 2.2e-7, 0.8 units in the last place rms (over [-9, 9], exp2 one unit off);
-// +-1 at infinity, NaN for NaN. Both branches are computed: 12 vector operations and two
-// transcendental ones, without divergence.
+// tanh in FP32, odd: x + x^3 P(x^2) below 1 (P: minimax polynomial of (tanh(x)/x - 1)/x^2, fitted for
+// this; 5e-9), 1 - 2 / (1 + exp(2 |x|)) with x's sign from the hardware exp2 and reciprocal above;
+// +-1 at infinity, NaN for NaN. Both branches are computed, without divergence. Against 64 bits, over
+// 8.4e6 arguments in [1e-8, 10] and their negatives: at most 1.22 units in the last place (7.3e-8),
+// 0.277 rms; tanhf 1.34 (8.0e-8) and 0.279, in 1.2 times the time. The line lies at 1 because the
+// exponential's error is larger just above it: at 0.8 the maximum is 1.40 (and 5 % less time), at 0.6
+// 1.59 (9 % less).
 __device__ inline float mlp_tanh(float x)
 {
 	const float ax = fabsf(x);
-	const float t  = __builtin_amdgcn_exp2f(2.88539008f * x);
+	const float t  = __builtin_amdgcn_exp2f(2.88539008f * ax);
 	const float m  = __builtin_amdgcn_rcpf(1.0f + t);
 	const float s  = x * x;
-	float       p  = -5.89515828e-3f;
-	p              = fmaf(p, s, 2.07959712e-2f);
-	p              = fmaf(p, s, -5.37838303e-2f);
-	p              = fmaf(p, s, 1.33319244e-1f);
-	p              = fmaf(p, s, -3.33332986e-1f);
+	float       p  = -3.58451944e-4f;
+	p              = fmaf(p, s, 2.30136444e-3f);
+	p              = fmaf(p, s, -7.94610567e-3f);
+	p              = fmaf(p, s, 2.14866567e-2f);
+	p              = fmaf(p, s, -5.38798012e-2f);
+	p              = fmaf(p, s, 1.33323446e-1f);
+	p              = fmaf(p, s, -3.33332956e-1f);
 	const float lo = fmaf(x * s, p, x);
-	const float hi = fmaf(-2.0f, m, 1.0f);
-	return ax < 0.6f ? lo : hi;
+	const float hi = copysignf(fmaf(-2.0f, m, 1.0f), x);
+	return ax < 1.0f ? lo : hi;
 }
 
 // The forward weights of one wave: left operands of both layers in registers; biases and W3

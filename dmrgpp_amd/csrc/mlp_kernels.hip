@@ -25,12 +25,12 @@ constexpr int kLd     = kMlpHidden + 4; // LDS row: 16-byte aligned, 4 banks fur
 
 // y[s] = MLP(x[s]) for count samples (features row major, kMlpIn per sample): each wave takes
 // tiles of 16 samples, grid-stride, the next tile's features loaded during the current one.
-// Bound by the vector ALU: 128 tanh per sample and the splits of layer 1's results, about 640
-// vector and 64 transcendental operations per tile (0.22 ms for 2.86e6 samples); the bf16 MFMAs
+// Bound by the vector ALU: 128 tanh per sample and the splits of layer 1's results, about 740
+// vector and 64 transcendental operations per tile (0.25 ms for 2.86e6 samples); the bf16 MFMAs
 // (52 per tile) run beside them, with three waves per SIMD. 2.86e6 samples, whole call: 4.97 ms
-// with one sample per thread (weights in LDS, activations in scratch), 0.38 ms with layer 2 on
-// FP32 MFMAs, 0.27 ms now; error of y against 64 bits 1.7e-7 before, 1.0e-7 now (features
-// N(0, 1), weights of a trained network's size).
+// with one sample per thread (weights in LDS, activations in scratch), 0.29 ms now (0.27 with a
+// tanh of 3.7 units in the last place); error of y against 64 bits, five networks of a trained
+// one's size on features N(0, 1): 1.7e-7 to 3.7e-7 with one sample per thread, 1.1e-7 to 2.7e-7 now.
 __global__ __launch_bounds__(kT) __attribute__((amdgpu_waves_per_eu(3))) void mlp_forward_kernel(
     const float* __restrict__ params, const float* __restrict__ x, int64_t count,
     float* __restrict__ y)

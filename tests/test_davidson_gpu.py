@@ -93,6 +93,31 @@ def test_gpu_mlp_forward_tiles(count):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("lo,hi", [(2.0 ** -60, 1e-3), (1e-3, 0.5), (0.5, 0.999), (0.999, 1.001), (1.001, 3.0),
+                                   (3.0, 20.0)])
+def test_gpu_mlp_activation(lo, hi):
+    """The activation on both sides of its line: layer 1's unit 0 is tanh(x0), which layer 2 keeps
+    exactly apart from a power of two (its unit is 2^-40 times that, where tanh is the identity, and
+    the smallest parts stay above FP32's smallest normal number).
+    Odd to the last bit, and within 1.5 units in the last place of 64-bit tanh (tanhf: 1.34)."""
+    n = 20000
+    v = np.exp(np.random.default_rng(8).uniform(np.log(lo), np.log(hi), n)).astype(np.float32)
+    x = np.zeros((2 * n, 4), dtype=np.float32)
+    x[:n, 0], x[n:, 0] = v, -v
+    p = np.zeros(mlp_oracle.NPARAMS, dtype=np.float32)
+    p[0] = 1.0
+    p[mlp_oracle.OFF_W2] = 2.0 ** -40
+    p[mlp_oracle.OFF_W3] = 2.0 ** 40
+    net = dm.Mlp(seed=5, capacity=1)
+    net.set_params(p)
+    y = net.forward(x)
+    net.close()
+    np.testing.assert_array_equal(y[n:], -y[:n])
+    want = np.tanh(v.astype(np.float64))
+    assert (np.abs(y[:n] - want) / np.spacing(want.astype(np.float32))).max() <= 1.5
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("count", [1, 17, 300])
 def test_gpu_mlp_forward_infinite_and_largest_weights(count):
     """Weights at the ends of FP32: an infinity times 0 is NaN, opposite ones cancel to NaN, one alone
@@ -102,7 +127,7 @@ def test_gpu_mlp_forward_infinite_and_largest_weights(count):
     # Hidden units of layer 1: 0 is exactly 0, 1 positive, 2 its negative; layer 2 unit 0 takes them.
     for weights, want in (((np.inf, 0, 0), np.nan), ((0, np.inf, 0), 1.0), ((0, -np.inf, 0), -1.0),
                           ((0, np.inf, np.inf), np.nan), ((np.nan, 0, 0), np.nan),
-                          ((big, 0, 0), 0.0), ((0, big, 0), 1.0)):
+                          ((big, 0, 0), 0.0), ((0, big, 0), 1.0), ((0, big, big), 0.0)):
         p = np.zeros(mlp_oracle.NPARAMS, dtype=np.float32)
         p[mlp_oracle.OFF_W1:mlp_oracle.OFF_B1].reshape(64, 4)[1:3, 0] = 1.0, -1.0
         p[mlp_oracle.OFF_W2:mlp_oracle.OFF_W2 + 3] = weights
