@@ -89,6 +89,10 @@ def test_gpu_mlp_forward_tiles(count):
     want = mlp_oracle.forward(p.astype(np.float64), f.astype(np.float64))[0]
     got = y[1:] if count > 64 else y
     assert np.all(np.abs(got - want) <= bound)
+    if count > 64:  # a sample of infinities: what numpy makes of it, and no other sample's affair
+        with np.errstate(invalid="ignore"):
+            first = mlp_oracle.forward(p.astype(np.float64), x[:1].astype(np.float64))[0]
+        assert np.isnan(first[0]) == np.isnan(y[0])
     net.close()
 
 

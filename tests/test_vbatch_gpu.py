@@ -115,9 +115,8 @@ def test_gpu_vbatch_alpha_zero_takes_any_contraction(cplx):
 @pytest.mark.parametrize("cplx", [False, True])
 @pytest.mark.parametrize("transa,transb", [("N", "N"), ("N", "T"), ("T", "N"), ("T", "T")])
 def test_gpu_vbatch_large_batch_tiles(transa, transb, cplx):
-    # Enough tiles for the 64 x 64 kernel (2048 of them), k at every remainder of a 16-element chunk
-    # and past the three chunks in flight, an odd base address; a few leading dimensions past the
-    # 32-bit offsets select the other variant.
+    # Enough tiles for the 64 x 64 kernel (2112 of them), k with and without a remainder of a 16-element
+    # chunk and past the four chunks in flight, an odd base address.
     rng = np.random.default_rng(3)
     w = 2 if cplx else 1
     dt = np.complex128 if cplx else np.float64
@@ -185,3 +184,47 @@ def test_gpu_vbatch_output_over_input_and_wide_rows(wide):
     np.testing.assert_array_equal(got[:m, n:], A[:, n:])
     if wide:
         np.testing.assert_array_equal(got[m:], X.reshape((ld, 4), order="F")[m:])
+
+
+@pytest.fixture(scope="module")
+def wide_buffers():
+    """Device memory for two matrices of 70 complex columns 2^21 + 3 apart."""
+    a, b = (dm.DeviceArray(2 * 70 * ((1 << 21) + 3)) for _ in range(2))
+    yield a, b
+    a.free()
+    b.free()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("transa,transb,cplx", [(a, b, c) for c in (False, True) for a in "NTC" for b in "NTC"
+                                                if c or "C" not in (a, b)])
+@pytest.mark.parametrize("count", [1, 1100])
+@pytest.mark.parametrize("wide", [False, True])
+@pytest.mark.parametrize("k", [4, 16, 70])
+def test_gpu_vbatch_tiles_and_offsets(wide_buffers, k, wide, count, transa, transb, cplx):
+    # 32- and 64-wide tiles (1 and 1100 tiles of 64 x 64) with 32- and 64-bit operand offsets (leading
+    # dimensions past 2^21), every transpose, alpha and beta, and contractions of a remainder
+    # alone, one whole chunk, and more chunks than are in flight with a remainder.
+    rng = np.random.default_rng(k)
+    w, dt = (2, np.complex128) if cplx else (1, np.float64)
+    alpha, beta = (0.5 - 0.25j, 2.0 + 1.0j) if cplx else (-0.5, 2.0)
+    m, n = 61, 63
+    stored = []
+    for dev, t, shape in zip(wide_buffers, (transa, transb), ((m, k), (k, n))):
+        r, c = shape if t == "N" else shape[::-1]
+        ld = (1 << 21) + 3 if wide else r + 1
+        x = rng.uniform(-1, 1, (c, r * w))  # by columns
+        for j in range(c):
+            dm._check(dm.lib().dmk_memcpy_h2d(dev.ptr + 8 * w * ld * j, x[j].ctypes.data, x[j].nbytes), "copy")
+        stored.append((dev.ptr, ld, _op(x.view(dt).T, t)))
+    (pa, lda, A), (pb, ldb, B) = stored
+    C = rng.uniform(-1, 1, (count, n, m * w))
+    dC = dm.DeviceArray.from_host(C.ravel())
+    dm.gemm_vbatch(transa, transb, [(m, n, k, lda, ldb, m, [(pa, pb, dC.ptr + e * C[0].nbytes)
+                                                            for e in range(count)])],
+                   alpha=alpha, beta=beta, cplx=cplx)
+    got = dC.download().view(dt).reshape(count, n, m)
+    want = alpha * (A @ B).T + beta * C.view(dt)
+    # k products of parts at most 1 (w of them to a part of the result), w k + 4 roundings each way,
+    # |alpha| < 1, and beta C at most 3 with four roundings.
+    assert np.abs(got - want).max() <= 2 * w * (w * k * (w * k + 4) + 16) * 2.0 ** -53
