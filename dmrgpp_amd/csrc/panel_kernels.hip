@@ -530,12 +530,8 @@ __global__ __launch_bounds__(kPThreads) void panel_gemm_kernel(
 				issue(A1, B1);
 				wait_vm_lgkm0<NW>();
 				barrier_no_fence();
-				int c = 0, left = kFoldSteps;
+				int c = 0;
 				for (; c + 3 <= nch; c += 3) {
-					if (kFold && --left < 0) {
-						fold();
-						left = kFoldSteps - 1;
-					}
 					issue(A2, B2);
 					compute(A0, B0);
 					wait_vm_lgkm0<NW>();
