@@ -840,20 +840,28 @@ Tuning default_tuning(int precision)
 // While the chip has only a few such tiles per CU, a launch is bounded by its longest tile's
 // chain of K chunks (each waits for its loads) and by idle CUs, so the smallest tiles with two
 // chunks in flight win by far; from a few tiles per CU on, operand traffic and per-tile overhead
-// count, and larger tiles with more residency (two LDS stages) win by less. Timed on Heisenberg
-// and Hubbard superblocks of m = 128 .. 3500 states, all tile shapes x split-k x load depths x
-// K chunks x MFMA forms; matvec in us with 64 x 64 tiles everywhere (the former choice), with the
-// rule, and with the best of all combinations (the K loop, the result stores and the LDS masks of the
-// kernels have since taken 1 to 5 % off all three; the largest BF16x3 problems have moved to 128 x 128):
-//            t1    t2    FP64                FP32                BF16x3
-//   spin 128   0.1  0.04    40 /   24 /   23    31 /   21 /   21    33 /   28 /   28
-//   spin 512   0.8  0.3     88 /   44 /   42    55 /   33 /   33    58 /   41 /   41
-//   Hub. 400   3.1  0.4    131 /   59 /   58    79 /   45 /   44    76 /   53 /   51
-//   spin 1024  4.5  0.8    254 /  185 /  182   145 /  110 /  105   106 /   84 /   84
-//   Hub. 1024  5.5  1.7    282 /  210 /  210   162 /  122 /  122   106 /   96 /   93
-//   spin 2048 17    3.1   1213 / 1130 / 1073   650 /  555 /  540   378 /  323 /  321
-//   Hub. 2048 24    3.6    969 /  895 /  865   526 /  470 /  451   352 /  303 /  299
-//   Hub. 3072 93    7.0   4323 / 4280 / 4218  2352 / 2200 / 2174  1501 / 1244 / 1244
+// count, and larger tiles with more residency (two LDS stages) win by less. Chosen from all tile
+// shapes x load depths x K chunks x MFMA forms on Heisenberg and Hubbard superblocks of m = 128 ..
+// 3500 states; matvec in us with the base tuning (the former choice) / with the rule, timed in turn:
+//              t1    t2    FP64          FP32          BF16x3
+//   spin 128    0.1  0.04    37 /   23     29 /   20     30 /   26
+//   spin 512    0.8  0.3    115 /   59     70 /   41     68 /   52
+//   Hub. 400    3.1  0.4     82 /   45     53 /   34     49 /   37
+//   spin 1024   4.5  0.8    237 /  189    141 /  113    101 /   93
+//   spin 1400   8.4  1.5    422 /  409    245 /  235    151 /  145
+//   Hub. 1024   5.5  1.7    266 /  216    166 /  132    104 /  100
+//   Hub. 1400  12    1.8    365 /  340    213 /  186    144 /  140
+//   spin 1700  12    2.1    735 /  668    385 /  331    221 /  212
+//   spin 1900  14    2.6    875 /  890    490 /  448    295 /  284
+//   Hub. 1700  17    2.7    583 /  581    365 /  298    226 /  220
+//   spin 2048  17    3.1   1145 / 1094    634 /  541    358 /  322
+//   Hub. 2048  24    3.6    880 /  881    509 /  448    333 /  303
+//   Hub. 2200        4.3   1802 / 1791   1014 /  977    611 /  526
+//   spin 2700  27    4.9   2087 / 2088   1169 / 1104    682 /  561
+//   Hub. 3072  93    7.0   4127 / 4145   2312 / 2072   1393 / 1126
+//   spin 3500  45    8.0   4231 / 4228   2373 / 2123   1330 / 1037
+// (One and the same shape, as FP64's from t2 = 4.2 on, differs by up to 1 % between two handles
+// here.) The autotuner finds up to 5 % more.
 Tuning Plan::rule_tuning(int precision) const
 {
 	double t1 = 0, t2 = 0;
@@ -871,11 +879,12 @@ Tuning Plan::rule_tuning(int precision) const
 		t.kchunk = kchunk;
 	};
 	if (precision == PREC_BF16X3) {
-		// Pieces of 1024 elements of k as in the base tuning, and its MFMA form: the FP32 accumulator
-		// of a piece then rounds as often as with the base shapes, and the results are the same
-		// bit for bit. Longer pieces are up to 12 % faster (spin 1024: 2048 elements 82 us, 1024
-		// 92; spin 2048: no split 308, 1024 314; Hub. 3072: 2048 elements 1068, 1024 1138) and
-		// err more (spin 2048: 5.06e-6 against 64 bits, 5.02e-6; spin 1024 5.18e-6, 5.17e-6).
+		// Pieces of 1024 elements of k as in the base tuning, in every class, so results do not
+		// depend on the class; and 16 x 16 x 32 MFMAs, up to 5 % faster than the base's 32 x 32 x 16
+		// ones, whose accumulators round twice as often. The error is the base tuning's (5.02e-6
+		// against 64 bits on spin 2048, 5.17e-6 on spin 1024). Longer pieces are up to 12 % faster
+		// (spin 1024: 2048 elements 82 us, 1024 92; spin 2048: no split 308, 1024 314; Hub. 3072:
+		// 2048 elements 1068, 1024 1138) and err more (spin 2048 5.06e-6, spin 1024 5.18e-6).
 		// A second set of accumulators, added to every 512 k, takes the registers of a wave per
 		// SIMD at 128 x 64 (spin 2048 318 -> 333 us) and a third of the speed at 128 x 128.
 		t.splitk = 1024;
@@ -957,9 +966,10 @@ void Plan::release_multi_sets()
 //   FP64     Hub. 400 (t2 0.4) x 8 131 / 130 / 207, spin 1024 (0.8) x 4 679 / 677 / 688, x 8 1404 /
 //            1265 / 1270, Hub. 1024 (1.7) x 3 633 / 628 / 668, x 8 1721 / 1588 / 1586, Hub. 1400
 //            (1.8) x 2 673 / 675 / 637, x 3 1017 / 990 / 983, x 4 1364 / 1255 / 1266, x 8 2766 /
-//            2415 / 2422, spin 1400 (1.5) x 8 3298 / 2941 / 2980, Hub. 2048 (3.6) x 8 7383 / 7049 / 7087
-//   BF16x3   spin 1024 x 8 440 / 384 / 443, Hub. 1024 x 4 311 / 261 / 310, Hub. 1400 x 8 907 / 779 /
-//            908, Hub. 2048 x 8 1915 / 1922 / 2186
+//            2415 / 2422, spin 1400 (1.5) x 8 3298 / 2941 / 2980, Hub. 2048 (3.6) x 8 7383 /
+//            7049 / 7087
+//   BF16x3   spin 1024 x 8 446 / 388 / 459, Hub. 1024 x 4 315 / 266 / 313, Hub. 1400 x 8 910 / 786 /
+//            947, Hub. 2048 x 8 1908 / 1919 / 2306
 // Padding: 128 x 128 tiles cover 1.2 to 1.5 times the area of 64 x 64 ones there, and 2.8 times on
 // Hub. 400, whose patches are 1 to 80 wide (BF16x3 x 12: 103 us with the single vector's tiles, 144
 // with 128 x 128; x 8, 128 x 64, 1.6 times: 79 and 94; FP64 x 16, 64 x 64 against 32 x 32, 1.8
@@ -1706,8 +1716,8 @@ Tuning Plan::autotune(const double* vin, double* vout, int iters)
 {
 	if (iters < 1)
 		throw std::invalid_argument("dmk_autotune: iters must be >= 1");
-	// Coordinate descent from the better of the mode's base and the rule's shapes: each launch parameter in turn takes every
-	// value with the others fixed, keeping the fastest; two passes.
+	// Coordinate descent from the better of the mode's base and the rule's shapes: each launch
+	// parameter in turn takes every value with the others fixed, keeping the fastest; two passes.
 	auto time_of = [&](const Tuning& t) {
 		retune(t);
 		double ms = 0;

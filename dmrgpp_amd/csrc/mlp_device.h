@@ -8,10 +8,11 @@
 // lane group g supplies its own units on the right and W2[o][those units] on the left. So nothing
 // goes through LDS between layers, and the whole W2 stays in registers.
 //
-// Inference multiplies layer 2 on bf16 MFMAs with every FP32 operand split exactly into three
-// bf16 parts (8 + 8 + 8 bits: h = bf16(v), m = bf16(v - h), l = v - h - m rounded) and the six
-// products down to 2^-17 of the leading one kept (l l, l m and m l, below 2^-25, are dropped),
-// accumulated in FP32. The reason is the issue port: on gfx950 an FP32 (or FP64) MFMA keeps the
+// Inference multiplies layer 2 on bf16 MFMAs with every finite FP32 operand split into three bf16
+// parts (8 + 8 + 8 bits: h = bf16(v), m = bf16(v - h), l = v - h - m) and the six products down to
+// 2^-17 of the leading one kept (l l, l m and m l, below 2^-25, are dropped), accumulated in FP32:
+// the error of a whole network is smaller than with FP32 sums in order (figures at the inference
+// kernel). An infinite weight has no parts; see MlpWeightsInfinite. The reason is the issue port: on gfx950 an FP32 (or FP64) MFMA keeps the
 // vector ALU from issuing for its whole duration (32 MFMAs and 128 FMAs, two waves per SIMD: 1.85
 // and 1.04 ms alone, 2.65 ms together), a bf16 MFMA does not (1.83 and 1.04 ms alone, 1.85
 // together), and the tanh work alone keeps the vector ALU busy.

@@ -3,10 +3,10 @@
 //
 // The reference expands its groups into per-entry arrays and hands them to MAGMA
 // *_vbatched_max_nocheck (or a BLAS loop). Here one launch computes the output tiles of all
-// entries straight from the caller's matrices (vbatch_kernels.hip); the host checks the
-// arguments and uploads the entries and the XCDs' tile lists in one copy. A batch in which some C overlaps an
-// operand's memory is computed into a workspace and copied back. The call is synchronous, like
-// the reference's.
+// entries straight from the caller's matrices (vbatch_kernels.hip); the host checks the arguments
+// and uploads the entries and the XCDs' tile lists (vbatch_plan.h) in one copy. A batch in which some
+// C overlaps an operand's memory is computed into a workspace and copied back. The call is
+// synchronous, like the reference's.
 #include "vbatch.h"
 
 #include "dmk_internal.h"

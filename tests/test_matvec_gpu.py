@@ -334,8 +334,8 @@ def test_gpu_balanced_launch_multi_vector(prec):
 def test_gpu_rule_shapes(size):
     # One patch of size x (size + 3) per class of the launch-shape rule (0.02 to 5.6 tiles of
     # 64 x 64 per CU): every precision against numpy with the modes' usual bounds, several vectors
-    # in one launch bitwise the single vector's, and FP64 outside 3 to 4.2 tiles per CU and
-    # BF16x3 bitwise the base tuning's.
+    # in one launch bitwise the single vector's, FP64 outside 3 to 4.2 tiles per CU bitwise the
+    # base tuning's, and BF16x3 the same in every class.
     rng = np.random.default_rng(size)
     L, R = size, size + 3
 
