@@ -2,6 +2,7 @@
 // of matrices, its size for packed operands, and that the XCDs' run lists hold every tile once.
 #include "vbatch_plan.h"
 
+#include <algorithm>
 #include <cstdio>
 #include <cstdlib>
 #include <random>
@@ -84,6 +85,28 @@ int main()
 	check(dmk::vb_ranges(many, 0, 0, 8).size() == 3, "packed operands: three ranges");
 	many[77777].c = many[5].b;
 	check(dmk::vb_outputs_meet_inputs(many, 0, 0, 8), "one C in a B among 10^5");
+
+	// 20000 products of matrices allocated one by one, in any order: nothing joins.
+	{
+		std::vector<size_t> slot(60000);
+		for (size_t i = 0; i < slot.size(); ++i)
+			slot[i] = i;
+		std::shuffle(slot.begin(), slot.end(), rng);
+		std::vector<dmk::VbEntry> apart;
+		for (size_t i = 0; i < 20000; ++i)
+			apart.push_back(entry(4096 * slot[3 * i], 4096 * slot[3 * i + 1], 4096 * slot[3 * i + 2], 40,
+			                      40, 40, 0));
+		std::vector<dmk::VbRange> r = dmk::vb_ranges(apart, 0, 0, 8);
+		check(r.size() == 60000, "matrices with gaps stay apart");
+		dmk::vb_sort_ranges(r);
+		bool sorted = true;
+		for (size_t i = 0; i < r.size(); ++i)
+			sorted = sorted && r[i].lo == reinterpret_cast<uintptr_t>(at(4096 * i)) && r[i].hi - r[i].lo == 12800;
+		check(sorted, "by lower end, every range once");
+		check(!dmk::vb_outputs_meet_inputs(apart, 0, 0, 8), "apart in any order");
+		apart[12345].c = apart[54].a + 1599;
+		check(dmk::vb_outputs_meet_inputs(apart, 0, 0, 8), "one C at the last element of an A");
+	}
 
 	for (int T : { 32, 64 })
 		for (int count : { 1, 7, 65, 4097, 40000 }) {
